@@ -41,6 +41,8 @@ constexpr int kMaxDevices = 64;
 constexpr int kChunkThreads = 1024;       // threads of a chunked-binning workgroup
 constexpr int kMaxChunkTiles = 16384;     // tiles whose two counters fit in 128 KB of LDS
 constexpr int kMaxRowsPerChunk = 124 * kChunkThreads;  // rows of one chunked-binning workgroup
+constexpr int64_t kChunkTarget = 1024;  // chunks a plan is cut into when its rows allow
+constexpr int kChunkAllChans = 4;       // channels of a continuum plan whose chunks span them all
 constexpr int kRowBlockRows = 8 * kChunkThreads;  // rows of a row-block binning workgroup
 
 // Packed geometry of one sample relative to a tile origin:
@@ -175,7 +177,7 @@ struct PlanDev {
   uint32_t *bin_start;              // [n_bins + 1]
   uint32_t *cur_prim, *cur_dup;     // [n_bins]
   uint32_t *gunit_start, *dunit_start;  // [n_bins + 1]
-  uint32_t *scan_tmp;               // block sums
+  uint32_t *scan_tmp;               // block sums of the index passes
   // records, three words each: {sample, packed grid geometry, packed
   // degrid geometry}; the third word is written for primary records only
   uint32_t *rec;                    // [max_records][3]
@@ -194,13 +196,15 @@ struct PlanDev {
   // (chan 0 when rows carry their own channel)
   unsigned long long *gmask, *dmask;  // [n_words]
   int64_t n_words, mask_words_per_chan;
-  // chunked binning: a chunk is rows_per_chunk rows of one channel
+  // chunked binning: a chunk is rows_per_chunk rows of one channel, or of
+  // every channel (chunk_all)
   int32_t chunked;                  // chunked binning possible for this plan
+  int32_t chunk_all;
   int32_t rows_per_chunk, chunks_per_chan;
   // per chunk and tile, the chunk's primary (chunk_hist) and duplicate
   // (chunk_dup) counts, each then replaced by the first slot of that run
-  uint32_t *chunk_hist;             // [n_chan * chunks_per_chan][ntu * ntv]
-  uint32_t *chunk_dup;              // [n_chan * chunks_per_chan][ntu * ntv]
+  uint32_t *chunk_hist;             // [chunk][ntu * ntv], chunks channel by channel
+  uint32_t *chunk_dup;              // [chunk][ntu * ntv]
   int32_t chunk_scatter;            // records written through per-chunk LDS cursors
   int32_t order_nb;                 // baselines per time step of time-major rows (1: row order)
   // row-block binning (rows carry their own channel): kRowBlockRows rows per
@@ -226,8 +230,6 @@ struct av_plan_host;  // defined in plan.hip
 
 // launch helpers shared by the translation units
 int launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
-int scan_exclusive_u32(const uint32_t *in, uint32_t *out, int64_t n,
-                       uint32_t *tmp, hipStream_t s);
 int prepare_tables(const PlanDev &d, const double *cgk, hipStream_t s);
 // grid.hip: overwrite-mode zeroing before a tile kernel (sums of weights and
 // split-bin tiles), and the per-unit sums of weights into sumwt after it
@@ -279,4 +281,4 @@ struct av_plan {
 int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u, int32_t n_v,
                 double cell_u, double cell_v, int32_t support, int32_t oversampling,
                 int32_t tile_u, int32_t tile_v, int32_t geometry, int32_t unit_cap, av_plan *p,
-                char *base, size_t *bytes);
+                char *base, size_t *bytes, bool compact = false);

@@ -1,4 +1,4 @@
-// common.hip -- error reporting, device info, fills, scans and the
+// common.hip -- error reporting, device info, fills and the
 // prolate-spheroidal table kernels of libavgrid.so.
 #include <cstdio>
 #include <mutex>
@@ -60,99 +60,6 @@ int launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s) {
   if (blocks > 8192) blocks = 8192;
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, s, p, v, n);
   AV_LAUNCH_CHECK("k_fill_u32");
-  return AV_OK;
-}
-
-// ------------------------------------------------------------- scan ----
-// Exclusive prefix sum of n uint32 values into out[0..n], out[n] = total.
-// Three passes: per-block local scan (4096 values per block), scan of the
-// block totals in one block, and a final add.
-constexpr int kScanThreads = 256;
-constexpr int kScanPerThread = 16;
-constexpr int kScanBlock = kScanThreads * kScanPerThread;
-
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *sh, uint32_t &total) {
-  // Hillis-Steele over blockDim.x (<= 1024) values in LDS.
-  int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int off = 1; off < (int)blockDim.x; off <<= 1) {
-    uint32_t add = t >= off ? sh[t - off] : 0u;
-    __syncthreads();
-    sh[t] += add;
-    __syncthreads();
-  }
-  uint32_t incl = sh[t];
-  total = sh[blockDim.x - 1];
-  __syncthreads();
-  return incl - v;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scan_local(const uint32_t *in, uint32_t *out,
-                                                             int64_t n, uint32_t *block_sums) {
-  __shared__ uint32_t sh[kScanThreads];
-  int64_t base = (int64_t)blockIdx.x * kScanBlock + (int64_t)threadIdx.x * kScanPerThread;
-  uint32_t vals[kScanPerThread];
-  uint32_t s = 0;
-#pragma unroll
-  for (int k = 0; k < kScanPerThread; ++k) {
-    int64_t i = base + k;
-    vals[k] = i < n ? in[i] : 0u;
-    s += vals[k];
-  }
-  uint32_t total;
-  uint32_t excl = block_exclusive_scan(s, sh, total);
-#pragma unroll
-  for (int k = 0; k < kScanPerThread; ++k) {
-    int64_t i = base + k;
-    if (i < n) out[i] = excl;
-    excl += vals[k];
-  }
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(1024) void k_scan_sums(uint32_t *block_sums, int64_t nblk,
-                                                    uint32_t *grand_total) {
-  __shared__ uint32_t sh[1024];
-  // each thread handles a contiguous run of ceil(nblk/1024) sums
-  int64_t per = (nblk + 1023) / 1024;
-  int64_t b0 = (int64_t)threadIdx.x * per;
-  uint32_t s = 0;
-  for (int64_t k = 0; k < per; ++k)
-    if (b0 + k < nblk) s += block_sums[b0 + k];
-  uint32_t total;
-  uint32_t excl = block_exclusive_scan(s, sh, total);
-  for (int64_t k = 0; k < per; ++k) {
-    if (b0 + k < nblk) {
-      uint32_t v = block_sums[b0 + k];
-      block_sums[b0 + k] = excl;
-      excl += v;
-    }
-  }
-  if (threadIdx.x == 0) *grand_total = total;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(uint32_t *out, int64_t n,
-                                                           const uint32_t *block_sums) {
-  int64_t base = (int64_t)blockIdx.x * kScanBlock;
-  uint32_t add = block_sums[blockIdx.x];
-  for (int k = threadIdx.x; k < kScanBlock; k += kScanThreads) {
-    int64_t i = base + k;
-    if (i < n) out[i] += add;
-  }
-}
-
-int scan_exclusive_u32(const uint32_t *in, uint32_t *out, int64_t n, uint32_t *tmp,
-                       hipStream_t s) {
-  int64_t nblk = (n + kScanBlock - 1) / kScanBlock;
-  if (nblk < 1) nblk = 1;
-  hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nblk), dim3(kScanThreads), 0, s, in, out, n,
-                     tmp);
-  AV_LAUNCH_CHECK("k_scan_local");
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, tmp, nblk, out + n);
-  AV_LAUNCH_CHECK("k_scan_sums");
-  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nblk), dim3(kScanThreads), 0, s, out, n, tmp);
-  AV_LAUNCH_CHECK("k_scan_add");
   return AV_OK;
 }
 

@@ -58,9 +58,16 @@ extern "C" int av_grid_noalloc(const double *uvw, int64_t n_rows, const double *
                                void *stream) {
   av_plan plan{};
   size_t bytes = 0;
+  // a plan that fits the scratch only in its most compact layout takes that
+  bool compact = false;
   int rc = plan_layout(n_rows, n_chan, n_img_chan, n_u, n_v, cell_u, cell_v, support,
                        oversampling, tile_u, tile_v, AV_GEOM_REFERENCE, 0, &plan, nullptr,
                        &bytes);
+  if (rc == AV_OK && bytes > kScratchBytes) {
+    compact = true;
+    rc = plan_layout(n_rows, n_chan, n_img_chan, n_u, n_v, cell_u, cell_v, support, oversampling,
+                     tile_u, tile_v, AV_GEOM_REFERENCE, 0, &plan, nullptr, &bytes, compact);
+  }
   if (rc) return rc;
   if (bytes > kScratchBytes)
     return fail(AV_ERR_INVALID, "av_grid_noalloc: this call's plan needs " +
@@ -72,7 +79,7 @@ extern "C" int av_grid_noalloc(const double *uvw, int64_t n_rows, const double *
   if ((rc = scratch_on_current_device(&base, &device))) return rc;
   if ((rc = plan_layout(n_rows, n_chan, n_img_chan, n_u, n_v, cell_u, cell_v, support,
                         oversampling, tile_u, tile_v, AV_GEOM_REFERENCE, 0, &plan, base,
-                        &bytes)))
+                        &bytes, compact)))
     return rc;
   plan.device = device;
   if ((rc = av_plan_set_uvw(&plan, uvw, freq, chan_map, nullptr, stream))) return rc;

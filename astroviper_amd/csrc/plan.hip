@@ -102,9 +102,9 @@ __device__ inline int64_t bin_of(const PlanDev &P, int tu, int tv, int ic) {
   return ((int64_t)tu * P.ntv + tv) * P.n_img_chan + ic;
 }
 
-__global__ void k_chan_setup(PlanDev P, const double *freq, const int32_t *chan_map) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= P.n_chan) return;
+// One channel's constants into the plan.
+__device__ inline void setup_channel(const PlanDev &P, const double *freq,
+                                     const int32_t *chan_map, int c) {
   double f = freq[c];
   P.freq[c] = f;
   // numpy: -(freq_chan * delta_lm[0] * n_uv[0]) / c   (standard_grid.py:298-299)
@@ -116,6 +116,11 @@ __global__ void k_chan_setup(PlanDev P, const double *freq, const int32_t *chan_
   else
     m = (P.n_img_chan == P.n_chan) ? c : 0;
   P.chan_map[c] = m;
+}
+
+__global__ void k_chan_setup(PlanDev P, const double *freq, const int32_t *chan_map) {
+  int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < P.n_chan) setup_channel(P, freq, chan_map, c);
 }
 
 // Records of one sample.  A grid-valid sample gets a primary record in the
@@ -217,14 +222,6 @@ __global__ __launch_bounds__(256) void k_count(PlanDev P) {
   }
 }
 
-__global__ void k_cursors(PlanDev P) {
-  int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= P.n_bins) return;
-  uint32_t s = P.bin_start[b];
-  P.cur_prim[b] = s;
-  P.cur_dup[b] = s + P.cnt_prim[b];
-}
-
 // One store per record: 12 bytes for a primary record, 8 for a duplicate
 // (degrid units cover the primary records of a bin only, so a duplicate's
 // degrid word is never read).
@@ -293,31 +290,60 @@ __global__ __launch_bounds__(256) void k_scatter(PlanDev P) {
 // A chunk is rows [r0, r0 + rows_per_chunk) of one channel.  Per tile it
 // counts primaries (chunk_hist) and duplicates (chunk_dup), 32 bits each.
 
-// Chunked pass 1: per-tile counts of one chunk, gathered in LDS.
-__global__ __launch_bounds__(kChunkThreads) void k_count_chunks(PlanDev P) {
+// Chunked pass 1: per-tile counts of one chunk, gathered in LDS.  The
+// workgroup first forms its channels' constants (every chunk of a channel
+// writes the same values), so no launch of their own precedes this one.  A
+// wavefront takes 64 consecutive rows of one channel at a time.
+template <bool ALL>
+__global__ __launch_bounds__(kChunkThreads) void k_count_chunks(PlanDev P, const double *freq,
+                                                                const int32_t *chan_map) {
   extern __shared__ uint32_t h[];  // [n_tiles] primaries, then [n_tiles] duplicates
   const int64_t w = blockIdx.x;
-  const int chan = (int)(w / P.chunks_per_chan);
-  const int64_t r0 = (w - (int64_t)chan * P.chunks_per_chan) * P.rows_per_chunk;
+  const int chan0 = ALL ? 0 : (int)(w / P.chunks_per_chan);
+  const int64_t r0 = (w - (int64_t)chan0 * P.chunks_per_chan) * P.rows_per_chunk;
   const int ntiles = P.ntu * P.ntv;
   uint32_t *hd = h + ntiles;
+  if (ALL) {
+    for (int c = threadIdx.x; c < P.n_chan; c += blockDim.x) setup_channel(P, freq, chan_map, c);
+  } else if (threadIdx.x == 0) {
+    setup_channel(P, freq, chan_map, chan0);
+  }
   for (int i = threadIdx.x; i < 2 * ntiles; i += blockDim.x) h[i] = 0u;
-  const ChanGeo cg = chan_geo(P, chan);
   __syncthreads();
-  for (int64_t row = r0 + threadIdx.x; row < r0 + P.rows_per_chunk; row += blockDim.x) {
+  const int nch = ALL ? P.n_chan : 1;
+  const uint32_t groups = (uint32_t)P.rows_per_chunk / 64u;  // 64-row groups of the chunk
+  const uint32_t waves = blockDim.x / 64u;
+  int chan = chan0;
+  uint32_t grp = threadIdx.x / 64u;
+  while (grp >= groups) {
+    grp -= groups;
+    ++chan;
+  }
+  ChanGeo cg = chan_geo(P, min(chan, P.n_chan - 1));
+  while (chan < chan0 + nch) {
+    const int64_t row = r0 + grp * 64u + __lane_id();
     ItemGeo g;
     g.gvalid = g.dvalid = false;
     if (row < P.n_rows) sample_geometry_at(P, row, cg, P.uvw[row * 3 + 0], P.uvw[row * 3 + 1], g);
     write_masks(P, row, chan, g.gvalid, g.dvalid);
-    if (!(g.gvalid || g.dvalid)) continue;
-    const RecPlan rp = record_plan(P, g);
-    if (rp.gprim) {
-      atomicAdd(&h[rp.tu * P.ntv + rp.tv], 1u);
-      for (int a = rp.tu0; a <= rp.tu1; ++a)
-        for (int b = rp.tv0; b <= rp.tv1; ++b)
-          if (a != rp.tu || b != rp.tv) atomicAdd(&hd[a * P.ntv + b], 1u);
+    if (g.gvalid || g.dvalid) {
+      const RecPlan rp = record_plan(P, g);
+      if (rp.gprim) {
+        atomicAdd(&h[rp.tu * P.ntv + rp.tv], 1u);
+        for (int a = rp.tu0; a <= rp.tu1; ++a)
+          for (int b = rp.tv0; b <= rp.tv1; ++b)
+            if (a != rp.tu || b != rp.tv) atomicAdd(&hd[a * P.ntv + b], 1u);
+      }
+      if (rp.dsep) atomicAdd(&h[rp.du_t * P.ntv + rp.dv_t], 1u);
     }
-    if (rp.dsep) atomicAdd(&h[rp.du_t * P.ntv + rp.dv_t], 1u);
+    grp += waves;
+    if (grp >= groups) {
+      do {
+        grp -= groups;
+        ++chan;
+      } while (grp >= groups);
+      if (ALL) cg = chan_geo(P, min(chan, P.n_chan - 1));
+    }
   }
   __syncthreads();
   uint32_t *dst = P.chunk_hist + w * ntiles, *dstd = P.chunk_dup + w * ntiles;
@@ -327,22 +353,54 @@ __global__ __launch_bounds__(kChunkThreads) void k_count_chunks(PlanDev P) {
   }
 }
 
+// The runs of tile t that image channel ic gathers, those of one segment
+// `seg` of `nseg`: segments split the row-chunks.  When image channels gather
+// several channels (continuum), a segment takes its runs row-chunk by
+// row-chunk, channel by channel within one: the channels of a row, which
+// share cache lines, then lie a run apart in the bin instead of a whole
+// channel's records apart.
+template <typename F>
+__device__ inline void chunk_runs(const PlanDev &P, int ic, int t, int seg, int nseg, F f) {
+  const int ntiles = P.ntu * P.ntv, K = P.chunks_per_chan;
+  const int k0 = (int)((int64_t)K * seg / nseg), k1 = (int)((int64_t)K * (seg + 1) / nseg);
+  if (P.chunk_all) {
+    for (int k = k0; k < k1; ++k) f((int64_t)k * ntiles + t);
+  } else if (P.n_img_chan < P.n_chan) {
+    for (int k = k0; k < k1; ++k)
+      for (int c = 0; c < P.n_chan; ++c)
+        if (P.chan_map[c] == ic) f(((int64_t)c * K + k) * ntiles + t);
+  } else {
+    for (int c = 0; c < P.n_chan; ++c) {
+      if (P.chan_map[c] != ic) continue;
+      for (int k = k0; k < k1; ++k) f(((int64_t)c * K + k) * ntiles + t);
+    }
+  }
+}
+
 // Chunked pass 2: the counts of every bin, summed over the chunks of the
-// channels that map to its image channel.
+// channels that map to its image channel.  A workgroup takes 64 tiles of one
+// image channel, a wavefront one segment of their runs: a
+// continuum bin has hundreds of runs, and one thread per bin leaves most of
+// the chip idle while it walks them.
+constexpr int kSegTiles = 64, kMaxSegs = 16;
 __global__ void k_chunk_totals(PlanDev P) {
-  const int ntiles = P.ntu * P.ntv;
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (int64_t)P.n_img_chan * ntiles) return;
-  const int ic = (int)(id / ntiles);
-  const int t = (int)(id - (int64_t)ic * ntiles);
+  __shared__ uint32_t part[2][kMaxSegs][kSegTiles];
+  const int nbt = (P.ntu * P.ntv + kSegTiles - 1) / kSegTiles;
+  const int ic = blockIdx.x / nbt, t = (blockIdx.x - ic * nbt) * kSegTiles + threadIdx.x;
+  const int seg = threadIdx.y, nseg = blockDim.y;
   uint32_t sp = 0, sd = 0;
-  for (int c = 0; c < P.n_chan; ++c) {
-    if (P.chan_map[c] != ic) continue;
-    for (int k = 0; k < P.chunks_per_chan; ++k) {
-      const int64_t i = ((int64_t)c * P.chunks_per_chan + k) * ntiles + t;
+  if (t < P.ntu * P.ntv)
+    chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
       sp += P.chunk_hist[i];
       sd += P.chunk_dup[i];
-    }
+    });
+  part[0][seg][threadIdx.x] = sp;
+  part[1][seg][threadIdx.x] = sd;
+  __syncthreads();
+  if (seg != 0 || t >= P.ntu * P.ntv) return;
+  for (int k = 1; k < nseg; ++k) {
+    sp += part[0][k][threadIdx.x];
+    sd += part[1][k][threadIdx.x];
   }
   const int64_t b = (int64_t)t * P.n_img_chan + ic;
   P.cnt_prim[b] = sp;
@@ -352,38 +410,36 @@ __global__ void k_chunk_totals(PlanDev P) {
 // Chunked pass 3 (after the bin offsets): the first slot of every chunk's
 // run in every bin.  The first primary slot overwrites the primary counts
 // (chunk_hist), the first duplicate slot the duplicate counts (chunk_dup).
-// When image channels gather several channels (continuum), a bin takes its
-// runs row-chunk by row-chunk, channel by channel within one: the channels
-// of a row, which share cache lines, then lie a run apart in the bin
-// instead of a whole channel's records apart.  Otherwise (one channel per
-// image channel) a bin takes its channel's runs in row order.
 __global__ void k_chunk_bases(PlanDev P) {
-  const int ntiles = P.ntu * P.ntv;
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (int64_t)P.n_img_chan * ntiles) return;
-  const int ic = (int)(id / ntiles);
-  const int t = (int)(id - (int64_t)ic * ntiles);
+  __shared__ uint32_t part[2][kMaxSegs][kSegTiles];
+  const int nbt = (P.ntu * P.ntv + kSegTiles - 1) / kSegTiles;
+  const int ic = blockIdx.x / nbt, t = (blockIdx.x - ic * nbt) * kSegTiles + threadIdx.x;
+  const int seg = threadIdx.y, nseg = blockDim.y;
+  const bool on = t < P.ntu * P.ntv;
+  uint32_t sp = 0, sd = 0;
+  if (on && nseg > 1)
+    chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
+      sp += P.chunk_hist[i];
+      sd += P.chunk_dup[i];
+    });
+  part[0][seg][threadIdx.x] = sp;
+  part[1][seg][threadIdx.x] = sd;
+  __syncthreads();
+  if (!on) return;
   const int64_t b = (int64_t)t * P.n_img_chan + ic;
-  uint32_t sp = P.bin_start[b];
-  uint32_t sd = sp + P.cnt_prim[b];
-  auto take = [&](int c, int k) {
-    const int64_t i = ((int64_t)c * P.chunks_per_chan + k) * ntiles + t;
+  sp = P.bin_start[b];
+  sd = sp + P.cnt_prim[b];
+  for (int k = 0; k < seg; ++k) {
+    sp += part[0][k][threadIdx.x];
+    sd += part[1][k][threadIdx.x];
+  }
+  chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
     const uint32_t np = P.chunk_hist[i], nd = P.chunk_dup[i];
     P.chunk_hist[i] = sp;
     P.chunk_dup[i] = sd;
     sp += np;
     sd += nd;
-  };
-  if (P.n_img_chan < P.n_chan) {
-    for (int k = 0; k < P.chunks_per_chan; ++k)
-      for (int c = 0; c < P.n_chan; ++c)
-        if (P.chan_map[c] == ic) take(c, k);
-  } else {
-    for (int c = 0; c < P.n_chan; ++c) {
-      if (P.chan_map[c] != ic) continue;
-      for (int k = 0; k < P.chunks_per_chan; ++k) take(c, k);
-    }
-  }
+  });
 }
 
 // Slots for one record per lane from the LDS cursors `cur` (key: the tile,
@@ -406,22 +462,36 @@ __device__ inline uint32_t run_slots(uint32_t *cur, int key) {
   return (uint32_t)__shfl((int)base, first) + (uint32_t)(lane - first);
 }
 
+// p / d for p, d < 2^32 by multiplication, with mul = ceil(2^32 / d):
+// the product's high word is p / d or one more.
+__device__ inline uint32_t div_by(uint32_t p, uint32_t d, uint64_t mul) {
+  uint32_t q = (uint32_t)(((uint64_t)p * mul) >> 32);
+  return (uint64_t)q * d > p ? q - 1 : q;
+}
+
 // Chunked pass 4: a workgroup per chunk writes the chunk's records.  Its
 // runs' first slots are loaded into LDS cursors, and the records take their
 // slots from LDS atomics, one per run of equal tiles in a wavefront: no
 // global atomics.  When the rows are time-major with order_nb baselines per
 // time step, the chunk's rows are visited baseline by baseline: a
 // wavefront then holds consecutive times of one baseline, which mostly fall
-// in the same tile, so its stores to a bin are contiguous.  (Numbering the
-// chunks so that 16, 32 or 64 consecutive chunks of a channel share an
-// XCD's L2 measured the same as plain numbering.)
+// in the same tile, so its stores to a bin are contiguous.  A chunk of every
+// channel (ALL) visits a row's channels before the next row: they mostly fall
+// in one tile, so a bin's records run through contiguous samples, and the
+// gridder's gathers and the degridder's stores are whole cache lines: on
+// 725,760 rows x 48 channels x 2 polarisations, one 1800 x 1500 plane per
+// polarisation, binning 1398 -> 969 us, the FP32 gridder 3788 -> 1421 us and
+// the degridder 1403 -> 1160 us, against chunks of one channel.
+// (Numbering the chunks so that 16, 32 or 64 consecutive chunks of a channel
+// share an XCD's L2 measured the same as plain numbering.)
+template <bool ALL>
 __global__ __launch_bounds__(kChunkThreads) void k_scatter_chunks(PlanDev P) {
   extern __shared__ uint32_t lds[];
   const int ntiles = P.ntu * P.ntv;
   uint32_t *cp = lds, *cd = lds + ntiles;  // [n_tiles] each
   const int64_t w = blockIdx.x;
-  const int chan = (int)(w / P.chunks_per_chan);
-  const int64_t r0 = (w - (int64_t)chan * P.chunks_per_chan) * P.rows_per_chunk;
+  const int chan0 = ALL ? 0 : (int)(w / P.chunks_per_chan);
+  const int64_t r0 = (w - (int64_t)chan0 * P.chunks_per_chan) * P.rows_per_chunk;
   const int64_t r1 = min(r0 + (int64_t)P.rows_per_chunk, P.n_rows);
   const uint32_t *bp = P.chunk_hist + w * ntiles, *bd = P.chunk_dup + w * ntiles;
   for (int i = threadIdx.x; i < ntiles; i += blockDim.x) {
@@ -430,23 +500,32 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_chunks(PlanDev P) {
   }
   __syncthreads();
   // positions p = b * nt + t over the nt time steps the chunk touches, row
-  // (t_lo + t) * nb + b; rows outside [r0, r1) are skipped (nb = 1: p = row - r0)
+  // (t_lo + t) * nb + b; rows outside [r0, r1) are skipped (nb = 1: p = row -
+  // r0).  With ALL, position q = p * n_chan + channel.
   const int64_t nb = P.order_nb;
   const int64_t t_lo = r0 / nb;
   const uint32_t nt = (uint32_t)((r1 - 1) / nb - t_lo + 1);
-  const uint32_t n_pos = nt * (uint32_t)nb;
-  const uint64_t nt_mul = ((1ull << 32) + nt - 1) / nt;  // floor(p * nt_mul / 2^32) - p / nt in {0, 1}
-  const ChanGeo cg = chan_geo(P, chan);
+  const uint32_t nch = ALL ? (uint32_t)P.n_chan : 1u;
+  const uint32_t n_pos = nt * (uint32_t)nb * nch;
+  const uint64_t nt_mul = ((1ull << 32) + nt - 1) / nt;
+  const uint64_t nch_mul = ((1ull << 32) + nch - 1) / nch;
+  ChanGeo cg = chan_geo(P, chan0);
   const uint32_t lane = __lane_id();
   for (uint32_t p0 = threadIdx.x - lane; p0 < n_pos; p0 += blockDim.x) {
-    const uint32_t p = p0 + lane;
+    uint32_t p = p0 + lane;
     int64_t row = -1;
+    int chan = chan0;
     if (p < n_pos) {
-      uint32_t b = (uint32_t)(((uint64_t)p * nt_mul) >> 32);
-      if (b * nt > p) --b;
+      if (ALL) {
+        const uint32_t q = div_by(p, nch, nch_mul);
+        chan = (int)(p - q * nch);
+        p = q;
+      }
+      const uint32_t b = div_by(p, nt, nt_mul);
       const int64_t r = (t_lo + (int64_t)(p - b * nt)) * nb + b;
       if (r >= r0 && r < r1) row = r;
     }
+    if (ALL) cg = chan_geo(P, chan);
     ItemGeo g;
     g.gvalid = g.dvalid = false;
     if (row >= 0) sample_geometry_at(P, row, cg, P.uvw[row * 3 + 0], P.uvw[row * 3 + 1], g);
@@ -585,39 +664,6 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_rows(PlanDev P) {
   }
 }
 
-// units per bin: grid units cover every bin (an empty bin still owns its
-// tile), degrid units only the primary records.
-__global__ void k_unit_counts(PlanDev P, uint32_t *nug, uint32_t *nud) {
-  int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= P.n_bins) return;
-  uint32_t cap = (uint32_t)P.unit_cap;
-  uint32_t na = P.cnt_all[b], np = P.cnt_prim[b];
-  nug[b] = na == 0 ? 1u : (na + cap - 1) / cap;
-  nud[b] = (np + cap - 1) / cap;
-}
-
-__global__ void k_units(PlanDev P) {
-  int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= P.n_bins) return;
-  uint32_t cap = (uint32_t)P.unit_cap;
-  uint32_t s = P.bin_start[b];
-  uint32_t na = P.cnt_all[b], np = P.cnt_prim[b];
-  uint32_t g0 = P.gunit_start[b], g1 = P.gunit_start[b + 1];
-  uint32_t ng = g1 - g0;
-  for (uint32_t k = 0; k < ng; ++k) {
-    uint32_t first = s + k * cap;
-    uint32_t cnt = na > k * cap ? min(cap, na - k * cap) : 0u;
-    uint32_t fl = (ng > 1 ? kUnitMulti : 0u) | (k == 0 ? kUnitFirst : 0u);
-    P.gunits[g0 + k] = make_uint4((uint32_t)b, first, cnt, fl);
-  }
-  uint32_t d0 = P.dunit_start[b], d1 = P.dunit_start[b + 1];
-  for (uint32_t k = 0; k < d1 - d0; ++k) {
-    uint32_t first = s + k * cap;
-    uint32_t cnt = min(cap, np - k * cap);
-    P.dunits[d0 + k] = make_uint4((uint32_t)b, first, cnt, 0u);
-  }
-}
-
 // Pair units: the bins of tiles 2j and 2j + 1 (along v) of pair p, and the
 // primary records of both.
 __device__ inline void pair_bins(const PlanDev &P, int64_t p, int64_t &b0, bool &has1,
@@ -631,29 +677,280 @@ __device__ inline void pair_bins(const PlanDev &P, int64_t p, int64_t &b0, bool 
   n = P.cnt_prim[b0] + (has1 ? P.cnt_prim[b0 + P.n_img_chan] : 0u);
 }
 
-__global__ void k_pair_counts(PlanDev P, uint32_t *npu) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P.n_pairs) return;
-  int64_t b0;
-  bool has1;
-  uint32_t n;
-  pair_bins(P, p, b0, has1, n);
-  const uint32_t cap = (uint32_t)P.unit_cap;
-  npu[p] = (n + cap - 1) / cap;
+// ---- bin offsets and work units --------------------------------------------
+// From the bins' counts: the offsets of their records, the grid units (every
+// bin has one, an empty bin still owns its tile), the degrid units (primary
+// records only) and the pair units, each an exclusive scan of a value formed
+// from the counts.  The scans run together: index_bins walks a range of bins
+// with the three running totals, index_pairs a range of pairs.
+
+// Exclusive scan of N values per thread over the workgroup; `total` gets the
+// sums.  sh: [16][N] LDS words.
+template <int N>
+__device__ inline void block_scan_n(uint32_t (&v)[N], uint32_t (&total)[N], uint32_t *sh) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwv = blockDim.x >> 6;
+  uint32_t in[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    in[k] = v[k];
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t o = __shfl_up(v[k], off);
+      if (lane >= off) v[k] += o;
+    }
+    if (lane == 63) sh[wave * N + k] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    uint32_t before = 0, all = 0;
+    for (int w = 0; w < nwv; ++w) {
+      const uint32_t s = sh[w * N + k];
+      before += w < wave ? s : 0u;
+      all += s;
+    }
+    v[k] += before - in[k];
+    total[k] = all;
+  }
+  __syncthreads();
 }
 
-__global__ void k_pair_units(PlanDev P) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P.n_pairs) return;
+__device__ inline void bin_values(const PlanDev &P, int64_t b, uint32_t (&v)[3]) {
+  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t na = P.cnt_all[b], np = P.cnt_prim[b];
+  v[0] = na;
+  v[1] = na == 0 ? 1u : (na + cap - 1) / cap;
+  v[2] = (np + cap - 1) / cap;
+}
+
+__device__ inline uint32_t pair_value(const PlanDev &P, int64_t p) {
   int64_t b0;
   bool has1;
   uint32_t n;
   pair_bins(P, p, b0, has1, n);
   const uint32_t cap = (uint32_t)P.unit_cap;
-  const uint32_t k0 = P.punit_start[p], nu = P.punit_start[p + 1] - k0;
-  const uint32_t b1 = has1 ? (uint32_t)(b0 + P.n_img_chan) : kNoBin;
-  for (uint32_t k = 0; k < nu; ++k)
-    P.punits[k0 + k] = make_uint4((uint32_t)b0, k * cap, min(cap, n - k * cap), b1);
+  return (n + cap - 1) / cap;
+}
+
+// Offsets, cursors and units of bins [b0, b1), whose preceding bins hold
+// `carry` records, grid units and degrid units (updated).
+__device__ inline void index_bins(const PlanDev &P, int64_t b0, int64_t b1, uint32_t (&carry)[3],
+                                  uint32_t *sh) {
+  const uint32_t cap = (uint32_t)P.unit_cap;
+  for (int64_t base = b0; base < b1; base += blockDim.x) {
+    const int64_t b = base + threadIdx.x;
+    const bool on = b < b1;
+    uint32_t v[3] = {0u, 0u, 0u}, n[3], total[3];
+    if (on) bin_values(P, b, v);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) n[k] = v[k];
+    block_scan_n<3>(v, total, sh);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      v[k] += carry[k];
+      carry[k] += total[k];
+    }
+    if (!on) continue;
+    const uint32_t np = P.cnt_prim[b], na = n[0];
+    P.bin_start[b] = v[0];
+    P.gunit_start[b] = v[1];
+    P.dunit_start[b] = v[2];
+    P.cur_prim[b] = v[0];
+    P.cur_dup[b] = v[0] + np;
+    for (uint32_t k = 0; k < n[1]; ++k) {
+      const uint32_t cnt = na > k * cap ? min(cap, na - k * cap) : 0u;
+      const uint32_t fl = (n[1] > 1 ? kUnitMulti : 0u) | (k == 0 ? kUnitFirst : 0u);
+      P.gunits[v[1] + k] = make_uint4((uint32_t)b, v[0] + k * cap, cnt, fl);
+    }
+    for (uint32_t k = 0; k < n[2]; ++k)
+      P.dunits[v[2] + k] = make_uint4((uint32_t)b, v[0] + k * cap, min(cap, np - k * cap), 0u);
+  }
+}
+
+// Pair units of pairs [p0, p1), preceded by `carry` units (updated).
+__device__ inline void index_pairs(const PlanDev &P, int64_t p0, int64_t p1, uint32_t &carry,
+                                   uint32_t *sh) {
+  const uint32_t cap = (uint32_t)P.unit_cap;
+  for (int64_t base = p0; base < p1; base += blockDim.x) {
+    const int64_t p = base + threadIdx.x;
+    const bool on = p < p1;
+    int64_t b0 = 0;
+    bool has1 = false;
+    uint32_t n = 0u;
+    if (on) pair_bins(P, p, b0, has1, n);
+    const uint32_t nu = (n + cap - 1) / cap;
+    uint32_t v[1] = {nu}, total[1];
+    block_scan_n<1>(v, total, sh);
+    const uint32_t k0 = v[0] + carry;
+    carry += total[0];
+    if (!on) continue;
+    P.punit_start[p] = k0;
+    const uint32_t b1 = has1 ? (uint32_t)(b0 + P.n_img_chan) : kNoBin;
+    for (uint32_t k = 0; k < nu; ++k)
+      P.punits[k0 + k] = make_uint4((uint32_t)b0, k * cap, min(cap, n - k * cap), b1);
+  }
+}
+
+__device__ inline void index_ends(const PlanDev &P, const uint32_t (&carry)[3]) {
+  if (threadIdx.x != 0) return;
+  P.bin_start[P.n_bins] = carry[0];
+  P.gunit_start[P.n_bins] = carry[1];
+  P.dunit_start[P.n_bins] = carry[2];
+}
+
+// Small plans: the totals (of a chunked plan), every offset and unit and the
+// chunks' first slots in one workgroup, where the seven launches of the
+// general path cost more than the work (a 128 x 128, 4-channel plan of 28,080
+// samples, binned in 21 launches: 85 us; in three: 32 us).
+__global__ __launch_bounds__(1024) void k_index_small(PlanDev P) {
+  __shared__ uint32_t sh[16 * 3];
+  if (P.chunked && !P.row_chan) {
+    for (int64_t b = threadIdx.x; b < P.n_bins; b += blockDim.x) {
+      const int t = (int)(b / P.n_img_chan), ic = (int)(b - (int64_t)t * P.n_img_chan);
+      uint32_t sp = 0, sd = 0;
+      chunk_runs(P, ic, t, 0, 1, [&](int64_t i) {
+        sp += P.chunk_hist[i];
+        sd += P.chunk_dup[i];
+      });
+      P.cnt_prim[b] = sp;
+      P.cnt_all[b] = sp + sd;
+    }
+    __syncthreads();
+  }
+  uint32_t carry[3] = {0u, 0u, 0u}, pc = 0u;
+  index_bins(P, 0, P.n_bins, carry, sh);
+  index_ends(P, carry);
+  if (P.n_pairs > 0) {
+    index_pairs(P, 0, P.n_pairs, pc, sh);
+    if (threadIdx.x == 0) P.punit_start[P.n_pairs] = pc;
+  }
+  if (P.chunk_scatter) {
+    __syncthreads();
+    for (int64_t b = threadIdx.x; b < P.n_bins; b += blockDim.x) {
+      const int t = (int)(b / P.n_img_chan), ic = (int)(b - (int64_t)t * P.n_img_chan);
+      uint32_t sp = P.bin_start[b], sd = sp + P.cnt_prim[b];
+      chunk_runs(P, ic, t, 0, 1, [&](int64_t i) {
+        const uint32_t np = P.chunk_hist[i], nd = P.chunk_dup[i];
+        P.chunk_hist[i] = sp;
+        P.chunk_dup[i] = sd;
+        sp += np;
+        sd += nd;
+      });
+    }
+  }
+}
+
+// General path: per-block sums (kIndexSpan bins or pairs a block), one
+// workgroup that scans them in place, then the offsets and units block by
+// block.  scan_tmp: [3][bin blocks] then [pair blocks].
+constexpr int kIndexSpan = 4096;
+__global__ __launch_bounds__(1024) void k_index_sums(PlanDev P, int nb_blocks) {
+  __shared__ uint32_t sh[16 * 3];
+  const bool pairs = (int)blockIdx.x >= nb_blocks;
+  const int64_t blk = pairs ? blockIdx.x - nb_blocks : blockIdx.x;
+  const int64_t i1 = min((blk + 1) * (int64_t)kIndexSpan, pairs ? P.n_pairs : P.n_bins);
+  uint32_t sum[3] = {0u, 0u, 0u}, total[3];
+  for (int64_t i = blk * kIndexSpan + threadIdx.x; i < i1; i += blockDim.x) {
+    if (pairs) {
+      sum[0] += pair_value(P, i);
+    } else {
+      uint32_t v[3];
+      bin_values(P, i, v);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) sum[k] += v[k];
+    }
+  }
+  block_scan_n<3>(sum, total, sh);
+  if (threadIdx.x != 0) return;
+  if (pairs) {
+    P.scan_tmp[3 * (int64_t)nb_blocks + blk] = total[0];
+  } else {
+    for (int k = 0; k < 3; ++k) P.scan_tmp[(int64_t)k * nb_blocks + blk] = total[k];
+  }
+}
+
+__global__ __launch_bounds__(1024) void k_index_scan(PlanDev P, int nb_blocks, int np_blocks) {
+  __shared__ uint32_t sh[16];
+  uint32_t ends[4];
+  for (int q = 0; q < 4; ++q) {
+    uint32_t *a = P.scan_tmp + (int64_t)q * nb_blocks;
+    const int n = q < 3 ? nb_blocks : np_blocks;
+    uint32_t carry = 0u;
+    for (int i0 = 0; i0 < n; i0 += blockDim.x) {
+      const int i = i0 + threadIdx.x;
+      uint32_t v[1] = {i < n ? a[i] : 0u}, total[1];
+      block_scan_n<1>(v, total, sh);
+      if (i < n) a[i] = v[0] + carry;
+      carry += total[0];
+    }
+    ends[q] = carry;
+  }
+  const uint32_t e3[3] = {ends[0], ends[1], ends[2]};
+  index_ends(P, e3);
+  if (P.n_pairs > 0 && threadIdx.x == 0) P.punit_start[P.n_pairs] = ends[3];
+}
+
+__global__ __launch_bounds__(1024) void k_index_apply(PlanDev P, int nb_blocks) {
+  __shared__ uint32_t sh[16 * 3];
+  if ((int)blockIdx.x >= nb_blocks) {
+    const int64_t blk = blockIdx.x - nb_blocks;
+    uint32_t carry = P.scan_tmp[3 * (int64_t)nb_blocks + blk];
+    index_pairs(P, blk * kIndexSpan, min((blk + 1) * (int64_t)kIndexSpan, P.n_pairs), carry, sh);
+    return;
+  }
+  const int64_t blk = blockIdx.x;
+  uint32_t carry[3];
+  for (int k = 0; k < 3; ++k) carry[k] = P.scan_tmp[(int64_t)k * nb_blocks + blk];
+  index_bins(P, blk * kIndexSpan, min((blk + 1) * (int64_t)kIndexSpan, P.n_bins), carry, sh);
+}
+
+// Segments of the chunk totals and bases passes: about eight runs each.
+static int chunk_segments(const PlanDev &d) {
+  const int64_t runs =
+      (int64_t)d.chunks_per_chan * (d.chunk_all ? 1 : d.n_chan) / d.n_img_chan;
+  return (int)std::max<int64_t>(
+      1, std::min<int64_t>(std::min<int64_t>(kMaxSegs, d.chunks_per_chan), runs / 8));
+}
+
+// Whether one workgroup indexes the plan: its bins and, for a chunked plan,
+// its runs are few enough that walking them takes less than the general
+// path's launches.
+static bool index_is_small(const PlanDev &d) {
+  const int64_t runs =
+      d.chunked && !d.row_chan
+          ? d.n_bins * d.chunks_per_chan *
+                (d.chunk_all ? 1 : (d.n_chan + d.n_img_chan - 1) / d.n_img_chan)
+          : 0;
+  return d.n_bins <= 4096 && runs <= 32768;
+}
+
+// Bin offsets, cursors and units from the bins' counts (small chunked plans:
+// from the chunks' counts).
+static int launch_index(const PlanDev &d, hipStream_t s) {
+  if (index_is_small(d)) {
+    hipLaunchKernelGGL(k_index_small, dim3(1), dim3(1024), 0, s, d);
+    AV_LAUNCH_CHECK("k_index_small");
+    return AV_OK;
+  }
+  const int64_t ntiles = (int64_t)d.ntu * d.ntv;
+  const dim3 sg((unsigned)((ntiles + kSegTiles - 1) / kSegTiles * d.n_img_chan));
+  const dim3 sb(kSegTiles, (unsigned)chunk_segments(d));
+  if (d.chunked && !d.row_chan) {
+    hipLaunchKernelGGL(k_chunk_totals, sg, sb, 0, s, d);
+    AV_LAUNCH_CHECK("k_chunk_totals");
+  }
+  const int nbb = (int)((d.n_bins + kIndexSpan - 1) / kIndexSpan);
+  const int npb = (int)((d.n_pairs + kIndexSpan - 1) / kIndexSpan);
+  hipLaunchKernelGGL(k_index_sums, dim3((unsigned)(nbb + npb)), dim3(1024), 0, s, d, nbb);
+  AV_LAUNCH_CHECK("k_index_sums");
+  hipLaunchKernelGGL(k_index_scan, dim3(1), dim3(1024), 0, s, d, nbb, npb);
+  AV_LAUNCH_CHECK("k_index_scan");
+  hipLaunchKernelGGL(k_index_apply, dim3((unsigned)(nbb + npb)), dim3(1024), 0, s, d, nbb);
+  AV_LAUNCH_CHECK("k_index_apply");
+  if (d.chunk_scatter) {
+    hipLaunchKernelGGL(k_chunk_bases, sg, sb, 0, s, d);
+    AV_LAUNCH_CHECK("k_chunk_bases");
+  }
+  return AV_OK;
 }
 
 // per-call tables: the FP32 kernel table; for every kernel offset, the FP64
@@ -713,14 +1010,36 @@ using namespace av;
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Rows of a chunk.  Every chunk is a workgroup of the two binning passes:
+// kChunkTarget of them in all keep the chip busy, but a chunk also reads and
+// writes a word per tile in each of four passes, so it has at least half a
+// sample per tile.  Chunks as long as kMaxRowsPerChunk left most CUs idle: a
+// 302,400-row, 16-channel plan of 1024 x 1024 was 48 workgroups and binned in
+// 611 us, 213 us in 1024 chunks (512: 199, 2048: 246, 4096: 270; a 129 M
+// sample plan of 2048 x 2048, already 1024 chunks, 2048 chunks: +12%).
+static int32_t chunk_rows(int64_t n_rows, int32_t n_chan, int64_t ntiles, bool all,
+                          bool compact) {
+  const int64_t per_row = all ? n_chan : 1;  // samples of a chunk per row
+  const int64_t step = all ? 64 : kChunkThreads;
+  int64_t rows = kMaxRowsPerChunk;
+  if (!compact)
+    rows = std::max((n_rows * n_chan / per_row + kChunkTarget - 1) / kChunkTarget,
+                    ntiles / 2 / per_row);
+  // a chunk's positions fit 32 bits
+  if (all) rows = std::min<int64_t>(rows, std::max<int64_t>(64, (1ll << 30) / n_chan));
+  rows = std::min<int64_t>({rows, n_rows, kMaxRowsPerChunk});
+  return (int32_t)(std::max<int64_t>(1, (rows + step - 1) / step) * step);
+}
+
 // Validate the plan parameters, fill plan->d's sizes and compute the bytes
 // of device memory the plan's arrays need; with base non-NULL, also point
 // the arrays into [base, base + bytes).  Shared by av_plan_create (one
-// hipMalloc) and av_grid_noalloc (the library's static scratch array).
+// hipMalloc) and av_grid_noalloc (the library's static scratch array).  With
+// `compact`, chunks are as long as they may be: the fewest bytes.
 int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u, int32_t n_v,
                 double cell_u, double cell_v, int32_t support, int32_t oversampling,
                 int32_t tile_u, int32_t tile_v, int32_t geometry, int32_t unit_cap, av_plan *p,
-                char *base, size_t *bytes) {
+                char *base, size_t *bytes, bool compact) {
   if (n_rows < 0 || n_chan < 1 || n_img_chan < 1 || n_u < 1 || n_v < 1)
     return fail(AV_ERR_INVALID, "av_plan_create: sizes must be positive");
   // plans bin footprints up to kMaxPlanSupport wide (the mosaic gridder's
@@ -743,9 +1062,9 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
     return fail(AV_ERR_INVALID, "av_plan_create: unknown geometry");
   if (conjugate && geometry != AV_GEOM_REFERENCE)
     return fail(AV_ERR_INVALID, "av_plan_create: AV_GEOM_CONJUGATE needs AV_GEOM_REFERENCE");
+  int64_t n_items = row_channels ? n_rows : n_rows * (int64_t)n_chan;
   if (unit_cap == 0) unit_cap = 8192;
   if (unit_cap < 64) return fail(AV_ERR_INVALID, "av_plan_create: unit_cap < 64");
-  int64_t n_items = row_channels ? n_rows : n_rows * (int64_t)n_chan;
   if (n_items > ((int64_t)1 << 32) / 5 - 1)
     return fail(AV_ERR_UNSUPPORTED, "av_plan_create: more than 858993458 samples per plan");
 
@@ -789,17 +1108,16 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.uvw = nullptr;
 
   const int64_t nb = d.n_bins;
-  int64_t scan_blocks = (std::max<int64_t>(nb, n_items) + 4095) / 4096 + 1;
   d.mask_words_per_chan = (n_rows + 63) / 64;
   const int64_t mask_words = d.mask_words_per_chan * (row_channels ? 1 : n_chan) + 1;
   // chunked binning when a channel's tiles fit in LDS
   const int64_t ntiles = (int64_t)d.ntu * d.ntv;
   d.chunked = !row_channels && ntiles <= kMaxChunkTiles && n_rows > 0;
-  d.rows_per_chunk = (int32_t)std::min<int64_t>(
-      kMaxRowsPerChunk, std::max<int64_t>(kChunkThreads,
-                                          (n_rows + kChunkThreads - 1) / kChunkThreads * kChunkThreads));
+  d.chunk_all = d.chunked && n_img_chan == 1 && n_chan >= kChunkAllChans && !compact;
+  d.rows_per_chunk = chunk_rows(n_rows, n_chan, ntiles, d.chunk_all, compact);
   d.chunks_per_chan = (int32_t)((n_rows + d.rows_per_chunk - 1) / d.rows_per_chunk);
-  const int64_t chunk_cells = d.chunked ? (int64_t)n_chan * d.chunks_per_chan * ntiles : 0;
+  const int64_t chunk_cells =
+      d.chunked ? (int64_t)(d.chunk_all ? 1 : n_chan) * d.chunks_per_chan * ntiles : 0;
   // row-block counts, kept for plans whose rows carry their channel when a
   // block's counters and cursors fit in 160 KB of LDS
   const int64_t row_cells = (row_channels && n_rows > 0 && 8 * ntiles <= 160 * 1024)
@@ -815,7 +1133,7 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
          o_freq = take(sizeof(double) * n_chan), o_cmap = take(sizeof(int32_t) * n_chan),
          o_call = take(4 * nb), o_cprim = take(4 * nb), o_bstart = take(4 * (nb + 1)),
          o_curp = take(4 * nb), o_curd = take(4 * nb), o_gus = take(4 * (nb + 1)),
-         o_dus = take(4 * (nb + 1)), o_scan = take(4 * scan_blocks),
+         o_dus = take(4 * (nb + 1)),
          o_rec = take(12 * std::max<int64_t>(d.max_records, 1)), o_gun = take(sizeof(uint4) * d.max_gunits),
          o_dun = take(sizeof(uint4) * d.max_dunits), o_pus = take(4 * (d.n_pairs + 1)),
          o_pun = take(sizeof(uint4) * d.max_punits),
@@ -840,7 +1158,6 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.cur_dup = (uint32_t *)(c + o_curd);
   d.gunit_start = (uint32_t *)(c + o_gus);
   d.dunit_start = (uint32_t *)(c + o_dus);
-  d.scan_tmp = (uint32_t *)(c + o_scan);
   d.rec = (uint32_t *)(c + o_rec);
   d.gunits = (uint4 *)(c + o_gun);
   d.dunits = (uint4 *)(c + o_dun);
@@ -857,6 +1174,9 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.wtab32 = (float *)(c + o_wt32);
   d.wtab64 = (double *)(c + o_wt64);
   d.upart = (double *)(c + o_upart);
+  // the index passes' block sums (four words per kIndexSpan bins at most):
+  // the units' partial sums are written after them, by the gridder
+  d.scan_tmp = (uint32_t *)d.upart;
   d.counters = (uint32_t *)(c + o_ctr);
   p->alloc_base = base;
   p->alloc_bytes = off;
@@ -918,11 +1238,7 @@ int av_plan_set_uvw(av_plan *plan, const double *uvw, const double *freq,
   if (row_chan) d.n_items = d.n_rows;  // one sample per row
   else d.n_items = d.n_rows * (int64_t)d.n_chan;
   d.n_words = d.mask_words_per_chan * (row_chan ? 1 : d.n_chan);
-  hipLaunchKernelGGL(k_chan_setup, dim3((d.n_chan + 255) / 256), dim3(256), 0, s, d, freq,
-                     chan_map);
-  AV_LAUNCH_CHECK("k_chan_setup");
   int rc;
-  const unsigned bb = (unsigned)((d.n_bins + 255) / 256);
   // row-block binning needs a counter and a cursor per tile in LDS
   const int64_t ntiles = (int64_t)d.ntu * d.ntv;
   d.row_blocks = 0;
@@ -934,78 +1250,64 @@ int av_plan_set_uvw(av_plan *plan, const double *uvw, const double *freq,
     if (row_chan) d.row_blocks = fits && d.row_hist != nullptr;
     else d.chunk_scatter = fits;
   }
-  const int64_t nchunks = (int64_t)d.n_chan * d.chunks_per_chan;
+  const int64_t nchunks = (int64_t)(d.chunk_all ? 1 : d.n_chan) * d.chunks_per_chan;
   const unsigned row_grid = (unsigned)((d.n_rows + kRowBlockRows - 1) / kRowBlockRows);
-  // pass 1: counts per bin
-  if (d.row_blocks) {
+  const bool by_chunks = d.chunked && !row_chan;
+  if (!by_chunks) {  // the counting pass of chunks sets its channels up itself
+    hipLaunchKernelGGL(k_chan_setup, dim3((d.n_chan + 255) / 256), dim3(256), 0, s, d, freq,
+                       chan_map);
+    AV_LAUNCH_CHECK("k_chan_setup");
     if ((rc = launch_fill_u32(d.cnt_all, 0u, d.n_bins, s))) return rc;
     if ((rc = launch_fill_u32(d.cnt_prim, 0u, d.n_bins, s))) return rc;
+  }
+  // pass 1: counts per bin, or per chunk and tile
+  if (d.row_blocks) {
     const int lds = (int)(sizeof(uint32_t) * ntiles);
     if ((rc = ensure_lds_limit<k_count_rows>(lds, "av_plan_set_uvw: hipFuncSetAttribute")))
       return rc;
     hipLaunchKernelGGL(k_count_rows, dim3(row_grid), dim3(kChunkThreads), lds, s, d);
     AV_LAUNCH_CHECK("k_count_rows");
-  } else if (d.chunked && !row_chan) {
-    const int lds = (int)(2 * sizeof(uint32_t) * d.ntu * d.ntv);
-    if ((rc = ensure_lds_limit<k_count_chunks>(lds, "av_plan_set_uvw: hipFuncSetAttribute")))
+  } else if (by_chunks) {
+    const int lds = (int)(2 * sizeof(uint32_t) * ntiles);
+    if ((rc = d.chunk_all ? ensure_lds_limit<k_count_chunks<true>>(
+                                lds, "av_plan_set_uvw: hipFuncSetAttribute")
+                          : ensure_lds_limit<k_count_chunks<false>>(
+                                lds, "av_plan_set_uvw: hipFuncSetAttribute")))
       return rc;
-    hipLaunchKernelGGL(k_count_chunks, dim3((unsigned)nchunks), dim3(kChunkThreads), lds, s, d);
+    hipLaunchKernelGGL(d.chunk_all ? k_count_chunks<true> : k_count_chunks<false>,
+                       dim3((unsigned)nchunks), dim3(kChunkThreads), lds, s, d, freq, chan_map);
     AV_LAUNCH_CHECK("k_count_chunks");
-    const int64_t pairs = (int64_t)d.n_img_chan * d.ntu * d.ntv;
-    hipLaunchKernelGGL(k_chunk_totals, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, s,
-                       d);
-    AV_LAUNCH_CHECK("k_chunk_totals");
   } else {
-    if ((rc = launch_fill_u32(d.cnt_all, 0u, d.n_bins, s))) return rc;
-    if ((rc = launch_fill_u32(d.cnt_prim, 0u, d.n_bins, s))) return rc;
     const int64_t span = d.mask_words_per_chan * 64 * (row_chan ? 1 : d.n_chan);
     int64_t blocks = (span + 255) / 256;
     blocks = std::max<int64_t>(1, std::min<int64_t>(blocks, 16384));
     hipLaunchKernelGGL(k_count, dim3((unsigned)blocks), dim3(256), 0, s, d);
     AV_LAUNCH_CHECK("k_count");
   }
-  // pass 2: bin offsets, cursors, records
-  if ((rc = scan_exclusive_u32(d.cnt_all, d.bin_start, d.n_bins, d.scan_tmp, s))) return rc;
+  // pass 2: bin offsets, cursors and units
+  if ((rc = launch_index(d, s))) return rc;
+  // pass 3: the records
   if (d.chunk_scatter) {
-    const int64_t pairs = (int64_t)d.n_img_chan * d.ntu * d.ntv;
-    hipLaunchKernelGGL(k_chunk_bases, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, s, d);
-    AV_LAUNCH_CHECK("k_chunk_bases");
     const int lds = (int)(2 * sizeof(uint32_t) * ntiles);
-    if ((rc = ensure_lds_limit<k_scatter_chunks>(lds, "av_plan_set_uvw: hipFuncSetAttribute")))
+    if ((rc = d.chunk_all ? ensure_lds_limit<k_scatter_chunks<true>>(
+                                lds, "av_plan_set_uvw: hipFuncSetAttribute")
+                          : ensure_lds_limit<k_scatter_chunks<false>>(
+                                lds, "av_plan_set_uvw: hipFuncSetAttribute")))
       return rc;
-    hipLaunchKernelGGL(k_scatter_chunks, dim3((unsigned)nchunks), dim3(kChunkThreads), lds, s, d);
+    hipLaunchKernelGGL(d.chunk_all ? k_scatter_chunks<true> : k_scatter_chunks<false>,
+                       dim3((unsigned)nchunks), dim3(kChunkThreads), lds, s, d);
     AV_LAUNCH_CHECK("k_scatter_chunks");
   } else if (d.row_blocks) {
-    hipLaunchKernelGGL(k_cursors, dim3(bb), dim3(256), 0, s, d);
-    AV_LAUNCH_CHECK("k_cursors");
     const int lds = (int)(2 * sizeof(uint32_t) * ntiles);
     if ((rc = ensure_lds_limit<k_scatter_rows>(lds, "av_plan_set_uvw: hipFuncSetAttribute")))
       return rc;
     hipLaunchKernelGGL(k_scatter_rows, dim3(row_grid), dim3(kChunkThreads), lds, s, d);
     AV_LAUNCH_CHECK("k_scatter_rows");
   } else {
-    hipLaunchKernelGGL(k_cursors, dim3(bb), dim3(256), 0, s, d);
-    AV_LAUNCH_CHECK("k_cursors");
     int64_t blocks = (d.n_items + 255) / 256;
     blocks = std::max<int64_t>(1, std::min<int64_t>(blocks, 16384));
     hipLaunchKernelGGL(k_scatter, dim3((unsigned)blocks), dim3(256), 0, s, d);
     AV_LAUNCH_CHECK("k_scatter");
-  }
-  // cursors are free again: reuse them for the per-bin unit counts
-  hipLaunchKernelGGL(k_unit_counts, dim3(bb), dim3(256), 0, s, d, d.cur_prim, d.cur_dup);
-  AV_LAUNCH_CHECK("k_unit_counts");
-  if ((rc = scan_exclusive_u32(d.cur_prim, d.gunit_start, d.n_bins, d.scan_tmp, s))) return rc;
-  if ((rc = scan_exclusive_u32(d.cur_dup, d.dunit_start, d.n_bins, d.scan_tmp, s))) return rc;
-  hipLaunchKernelGGL(k_units, dim3(bb), dim3(256), 0, s, d);
-  AV_LAUNCH_CHECK("k_units");
-  if (d.n_pairs > 0) {
-    // the bins' cursors are free again: the pairs' unit counts
-    const unsigned pb = (unsigned)((d.n_pairs + 255) / 256);
-    hipLaunchKernelGGL(k_pair_counts, dim3(pb), dim3(256), 0, s, d, d.cur_prim);
-    AV_LAUNCH_CHECK("k_pair_counts");
-    if ((rc = scan_exclusive_u32(d.cur_prim, d.punit_start, d.n_pairs, d.scan_tmp, s))) return rc;
-    hipLaunchKernelGGL(k_pair_units, dim3(pb), dim3(256), 0, s, d);
-    AV_LAUNCH_CHECK("k_pair_units");
   }
   return AV_OK;
 }

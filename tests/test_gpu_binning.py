@@ -1,0 +1,78 @@
+"""GPU binning where its passes change: one workgroup or several for the bin
+offsets, chunks of one channel or of all, one or many chunks and segments,
+and units shorter than a dense tile's records.
+
+A misplaced, lost or doubled record is an O(1) error of the grid or the
+model, so the FP64 bars of the parity tests (1e-12) apply."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+C = 299792458.0
+
+
+def _rel(a, b):
+    return float(np.max(np.abs(a - b)) / np.max(np.abs(b)))
+
+
+def _samples(nt, nb, nchan, npol, n_uv, seed, spread=0.45):
+    """Random uvw within `spread` of the grid's half width (some beyond it)."""
+    rng = np.random.default_rng(seed)
+    freq = np.linspace(1.0e9, 1.3e9, nchan)
+    cell = 1e-4
+    reach = spread * 2.2 * C / (2 * freq[-1] * cell)
+    uvw = rng.uniform(-reach, reach, size=(nt, nb, 3))
+    shape = (nt, nb, nchan, npol)
+    vis = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    w = rng.uniform(0.5, 1.5, size=shape)
+    flag = rng.random(shape) < 0.1
+    return uvw, freq, vis, w, flag, (-cell, cell)
+
+
+def _run(gpu, uvw, freq, vis, w, flag, n_uv, cell, cube, n_baseline, **plan_args):
+    from astroviper_amd.device import GridPlan
+    nt, nb, nchan, npol = w.shape
+    rows = nt * nb
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(rows, nchan, nchan if cube else 1, n_uv, cell, device=gpu,
+                    n_baseline=n_baseline, **plan_args)
+    plan.set_uvw(dev(uvw.reshape(rows, 3)), dev(freq))
+    flat = (rows * nchan, npol)
+    fl = dev(flag.reshape(flat).astype(np.uint8))
+    g, sw = plan.grid(dev(vis.reshape(flat)), dev(w.reshape(flat)), fl)
+    m = plan.degrid(g, fl)
+    st = plan.stats()
+    out = (g.cpu().numpy(), sw.cpu().numpy(), m.cpu().numpy(), st)
+    plan.close()
+    return out
+
+
+# (times, baselines, channels, n_u, n_v, cube): bins = tiles x image channels
+@pytest.mark.parametrize("nt,nb,nchan,n_u,n_v,cube", [
+    (1, 1, 1, 16, 16, True),          # one bin, one sample
+    (3, 21, 1, 64, 48, False),        # 63 rows: one partial mask word
+    (4, 16, 4, 512, 512, True),       # 4096 bins: the last single-workgroup plan
+    (4, 16, 4, 512, 528, True),       # 4224 bins: the general passes
+    (40, 351, 4, 96, 112, False),     # chunks of all channels, rows in order
+    (40, 351, 3, 96, 112, False),     # below the channels such chunks need
+    (60, 45, 48, 160, 160, False),    # several chunks, runs of 48 channels
+    (33, 67, 5, 1040, 1040, False),   # 4225 tiles: general passes, all channels
+    (33, 67, 9, 1040, 1024, True),    # several blocks of bins per channel
+])
+def test_binning_paths_match_oracle(gpu, oracle, nt, nb, nchan, n_u, n_v, cube):
+    n_uv = (n_u, n_v)
+    uvw, freq, vis, w, flag, cell = _samples(nt, nb, nchan, 2, n_uv, nt * nb + nchan)
+    w0 = np.where(flag, 0.0, w)
+    gref, swref = oracle.standard_grid(vis, uvw, w0, freq, n_uv, cell,
+                                       chan_mode="cube" if cube else "continuum")
+    for n_baseline in (nb, 1):
+        g, sw, m, st = _run(gpu, uvw, freq, vis, w, flag, n_uv, cell, cube, n_baseline)
+        mref = oracle.degrid(uvw, flag, freq, gref, cell)
+        if np.max(np.abs(gref)) > 0:
+            assert _rel(g, gref) < 1e-12
+            assert _rel(sw, swref) < 1e-12
+            assert _rel(m.reshape(mref.shape), mref) < 1e-12
+        assert st["grid_units"] >= st["bins"]
