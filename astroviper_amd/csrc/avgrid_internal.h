@@ -42,7 +42,8 @@ constexpr int kChunkThreads = 1024;       // threads of a chunked-binning workgr
 constexpr int kMaxChunkTiles = 16384;     // tiles whose two counters fit in 128 KB of LDS
 constexpr int kMaxRowsPerChunk = 124 * kChunkThreads;  // rows of one chunked-binning workgroup
 constexpr int64_t kChunkTarget = 1024;  // chunks a plan is cut into when its rows allow
-constexpr int kChunkAllChans = 4;       // channels of a continuum plan whose chunks span them all
+constexpr int kChunkAllChans = 2;       // channels of a continuum plan whose chunks span them all
+constexpr int64_t kCapSamples = 12288;  // samples of a plan per record of its default unit cap
 constexpr int kRowBlockRows = 8 * kChunkThreads;  // rows of a row-block binning workgroup
 
 // Packed geometry of one sample relative to a tile origin:
@@ -231,10 +232,11 @@ struct av_plan_host;  // defined in plan.hip
 // launch helpers shared by the translation units
 int launch_fill_u32(uint32_t *p, uint32_t v, int64_t n, hipStream_t s);
 int prepare_tables(const PlanDev &d, const double *cgk, hipStream_t s);
-// grid.hip: overwrite-mode zeroing before a tile kernel (sums of weights and
-// split-bin tiles), and the per-unit sums of weights into sumwt after it
-int zero_before_grid(const PlanDev &d, void *grid, int npol, bool fp64, double *sumwt,
-                     hipStream_t s);
+// grid.hip: before a tile kernel the call's tables (cgk given) and the zeros
+// of overwrite mode (grid given: sums of weights and split-bin tiles), and
+// the per-unit sums of weights into sumwt after it
+int prepare_grid(const PlanDev &d, const double *cgk, void *grid, int npol, bool fp64,
+                 double *sumwt, hipStream_t s);
 int reduce_sumwt(const PlanDev &d, int npol, double *sumwt, hipStream_t s);
 
 // properties of the current device, queried once per device

@@ -26,6 +26,8 @@ namespace av {
 constexpr int kGridThreads = 256;
 constexpr int kGridMaxWaves = kGridThreads / 64;
 constexpr int kCompChunkBatches = 4;  // compensated mode: fold every 4*64 records
+// compensated mode: records a workgroup sums, however short the plan's units
+constexpr uint32_t kCompGroupRecords = 8192;
 constexpr int kGridXcdGroup = 16;     // matrix-core kernel: workgroups per XCD group
 constexpr int kGridSubtile = AV_GRID_SUBTILE;
 
@@ -113,6 +115,36 @@ __device__ inline uint2 load_record(const PlanDev &P, uint32_t idx, uint32_t end
   return make_uint2(v.x, v.y);
 }
 
+// Compensated mode: the FP64 sums of split bins.  They lie in the unused end
+// of the plan's record array, one slot per kCompGroupRecords records: a bin
+// split into several groups holds more records than that, so
+// bin_start / kCompGroupRecords numbers its slot uniquely.  A sample has at
+// most four records (five with a degrid record of its own) of the five the
+// array has room for, and a slot at most 16 KB, two bytes per record, so the
+// slots fit whenever no sample has five; where they do not,
+// the groups add into the grid in FP32.
+__device__ inline double *comp_slots(const PlanDev &P, int slot_bytes) {
+  const uint64_t n_rec = P.bin_start[P.n_bins];
+  const uint64_t used = (n_rec * 12 + 255) & ~(uint64_t)255;
+  const uint64_t need = (n_rec / kCompGroupRecords + 1) * (uint64_t)slot_bytes;
+  return used + need <= (uint64_t)P.max_records * 12 ? (double *)((char *)P.rec + used) : nullptr;
+}
+
+// Compensated mode: the units of a bin are summed in groups of
+// kCompGroupRecords records.  True when unit {b, first} leads its group, of
+// n_in units and cnt records; `multi` when its bin has other groups.
+__device__ inline bool comp_group(const PlanDev &P, int64_t b, uint32_t first, uint32_t &n_in,
+                                  uint32_t &cnt, bool &multi) {
+  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t per = max(1u, kCompGroupRecords / cap);
+  const uint32_t k = (first - P.bin_start[b]) / cap;
+  const uint32_t n_units = P.gunit_start[b + 1] - P.gunit_start[b];
+  n_in = min(per, n_units - k);
+  cnt = min(n_in * cap, P.cnt_all[b] - k * cap);
+  multi = n_units > per;
+  return k % per == 0;
+}
+
 template <typename R, int NPOL, int DVW, bool COMP>
 __global__ __launch_bounds__(kGridThreads) void k_grid_tiles(PlanDev P, const R *__restrict__ vis,
                                                              const R *__restrict__ weight,
@@ -160,7 +192,16 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_tiles(PlanDev P, const R 
 
   const uint4 unit = P.gunits[u];
   const int64_t b = unit.x;
-  const uint32_t first = unit.y, cnt = unit.z, fl = unit.w;
+  const uint32_t first = unit.y;
+  uint32_t cnt = unit.z;
+  bool multi = (unit.w & kUnitMulti) != 0;
+  if (COMP) {  // the group's first unit walks the whole group
+    uint32_t n_in;
+    if (!comp_group(P, b, first, n_in, cnt, multi)) {
+      if (lane < NPOL) P.upart[(size_t)u * 4 + lane] = 0.0;
+      return;
+    }
+  }
   // 32-bit divisions: bins are numbered below 2^32 (64-bit ones cost
   // about a hundred scalar instructions each)
   const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
@@ -317,7 +358,6 @@ __global__ __launch_bounds__(kGridThreads) void k_grid_tiles(PlanDev P, const R 
   }
 
   // ---- flush the tile
-  const bool multi = (fl & kUnitMulti) != 0;
   if (COMP) {
 #pragma unroll
     for (int k = 0; k < kCpt; ++k) {
@@ -462,6 +502,48 @@ __device__ inline void copy_wtab_padded(R *w, const MfmaLds &L, const PlanDev &P
   }
 }
 
+// LDS in which a compensated group's wavefronts add their tiles in FP64, and
+// the size of a split bin's FP64 slot.
+template <int NPOL, int MB, int VB, bool COMP>
+__host__ __device__ constexpr int mfma_comb_bytes() {
+  return COMP ? MB * 2 * NPOL * VB * 4 * 64 * (int)sizeof(double) : 0;
+}
+
+// A wavefront's tile to the grid: lane l holds rows MfmaOp::row(l / 16, r),
+// column l % 16 of every block.
+template <typename R, int NPOL, int MB, int VB>
+__device__ inline void store_tile(const PlanDev &P,
+                                  const typename MfmaOp<R>::V (&acc)[MB][2 * NPOL][VB], R *gplane,
+                                  int u0, int v0, bool multi, bool accumulate) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const size_t pstride = (size_t)P.n_u * P.n_v * 2;
+#pragma unroll
+  for (int m = 0; m < MB; ++m)
+#pragma unroll
+    for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gu = u0 + 16 * m + MfmaOp<R>::row(lk, r), gv = v0 + 16 * vb + li;
+        if (gu >= P.n_u || gv >= P.n_v) continue;
+#pragma unroll
+        for (int p = 0; p < NPOL; ++p) {
+          const R re = acc[m][2 * p][vb][r], im = acc[m][2 * p + 1][vb][r];
+          R *dst = gplane + p * pstride + ((size_t)gu * P.n_v + gv) * 2;
+          if (multi) {
+            if (re != (R)0) atomicAdd(dst, re);
+            if (im != (R)0) atomicAdd(dst + 1, im);
+          } else if (accumulate) {
+            Cplx<R> old = *(Cplx<R> *)dst;
+            old.re += re;
+            old.im += im;
+            *(Cplx<R> *)dst = old;
+          } else {
+            *(Cplx<R> *)dst = Cplx<R>{re, im};
+          }
+        }
+      }
+}
+
 // Workgroups per CU the FP32 kernels with up to 8 result blocks are compiled
 // for: six (80 registers, no spills; a 16 x 16 tile's workgroup needs 26 KB
 // of LDS).  Other variants keep the compiler's choice.
@@ -499,19 +581,29 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
 
   const uint32_t n_units = P.gunit_start[P.n_bins];
   // 16 workgroups of 4 units: the 64 channels of a tile under one L2
-  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup);
-  if (blk * kGridMaxWaves >= n_units) return;  // whole workgroup idle
+  // (compensated: a workgroup per unit, that of a group's first unit sums the
+  // whole group)
+  constexpr int kUnitsPerWg = COMP ? 1 : kGridMaxWaves;
+  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup * kGridMaxWaves / kUnitsPerWg);
+  if (blk * kUnitsPerWg >= n_units) return;  // whole workgroup idle
   copy_wtab_padded(tab, L, P);
   for (int i = tid; i < L.nnrm; i += blockDim.x) nrm[i] = P.nrm[i];
   __syncthreads();  // the only workgroup barrier: tables ready
   // the same for every lane: scalar registers for the unit and its bounds
-  const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blk * kGridMaxWaves + wave));
+  uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)(COMP ? blk : blk * kGridMaxWaves + wave));
   if (u >= n_units) return;
 
   const int Tu = 16 * MB, Tv = 16 * VB;
   const uint4 unit = P.gunits[u];
   const int64_t b = unit.x;
-  const uint32_t first = unit.y, cnt = unit.z, fl = unit.w;
+  uint32_t first = unit.y, cnt = unit.z;
+  bool multi = (unit.w & kUnitMulti) != 0;
+  uint32_t n_in = 1;
+  if (COMP) {
+    if (!comp_group(P, b, first, n_in, cnt, multi)) return;
+    if (wave >= (int)n_in && n_in == 1) return;
+  }
   // 32-bit divisions: bins are numbered below 2^32 (64-bit ones cost
   // about a hundred scalar instructions each)
   const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
@@ -572,11 +664,18 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
             acc[m][c][vb][r] = reset ? (R)0 : t + ccmp[k];
           }
   };
+  // wavefronts of a compensated group take its units in turn
+  const uint32_t gend = first + cnt, lead = u;
+  for (uint32_t w = COMP ? (uint32_t)wave : 0u; w < n_in; w += kGridMaxWaves) {
+  if (COMP) {
+    u = lead + w;
+    first = unit.y + w * (uint32_t)P.unit_cap;
+  }
   double sw[NPOL];
 #pragma unroll
   for (int p = 0; p < NPOL; ++p) sw[p] = 0.0;
 
-  const uint32_t end = first + cnt;
+  const uint32_t end = COMP ? min(gend, first + (uint32_t)P.unit_cap) : gend;
   uint2 r0 = load_record(P, first + lane, end), r1 = load_record(P, first + 64 + lane, end);
   RawSample<R, NPOL> raw0;
   fetch_raw<R, NPOL>(raw0, r0.x, vis, weight, flag, psf, adjoint);
@@ -687,41 +786,98 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
     r0 = r1;
     r1 = r2;
   }
-  if (COMP) fold(false);
-
-  // ---- flush: lane holds rows MO::row(lane/16, r), column lane%16 of every block
-  const bool multi = (fl & kUnitMulti) != 0;
-#pragma unroll
-  for (int m = 0; m < MB; ++m)
-#pragma unroll
-    for (int vb = 0; vb < VB; ++vb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gu = u0 + 16 * m + MO::row(lk, r), gv = v0 + 16 * vb + li;
-        if (gu >= P.n_u || gv >= P.n_v) continue;
-#pragma unroll
-        for (int p = 0; p < NPOL; ++p) {
-          const R re = acc[m][2 * p][vb][r], im = acc[m][2 * p + 1][vb][r];
-          R *dst = gplane + p * pstride + ((size_t)gu * P.n_v + gv) * 2;
-          if (multi) {
-            if (re != (R)0) atomicAdd(dst, re);
-            if (im != (R)0) atomicAdd(dst + 1, im);
-          } else if (accumulate) {
-            Cplx<R> old = *(Cplx<R> *)dst;
-            old.re += re;
-            old.im += im;
-            *(Cplx<R> *)dst = old;
-          } else {
-            *(Cplx<R> *)dst = Cplx<R>{re, im};
-          }
-        }
-      }
   // ---- sums of weights (FP64): this unit's partial per polarisation
 #pragma unroll
   for (int p = 0; p < NPOL; ++p) {
     double sv = adjoint ? 0.0 : sw[p];
     for (int off = 32; off >= 1; off >>= 1) sv += __shfl_xor(sv, off);
     if (lane == 0) P.upart[(size_t)u * 4 + p] = sv;
+  }
+  if (COMP) fold(w + kGridMaxWaves < n_in);
+  }
+  if constexpr (COMP) {
+    if (n_in > 1) {
+      // the wavefronts' (sum, compensation) pairs, added in FP64 through LDS
+      double *comb = (double *)(smem + L.total);  // [kNc][64]
+      const int nwv = min(kGridMaxWaves, (int)n_in);
+      for (int w = 0; w < nwv; ++w) {
+        if (wave == w) {
+#pragma unroll
+          for (int k = 0; k < kNc; ++k) {
+            const double x = (double)csum[k] + (double)ccmp[k];
+            comb[k * 64 + lane] = w == 0 ? x : comb[k * 64 + lane] + x;
+          }
+        }
+        __syncthreads();
+      }
+      if (wave != 0) return;
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+          for (int vb = 0; vb < VB; ++vb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              acc[m][c][vb][r] = (R)comb[(((m * C + c) * VB + vb) * 4 + r) * 64 + lane];
+    }
+  }
+
+  // ---- flush: lane holds rows MO::row(lane/16, r), column lane%16 of every block
+  if constexpr (COMP) {
+    // a bin of several groups: into its FP64 slot, which k_comp_finish rounds
+    // to the grid once
+    double *slots = multi ? comp_slots(P, mfma_comb_bytes<NPOL, MB, VB, true>()) : nullptr;
+    if (slots) {
+      const double *comb = (const double *)(smem + L.total);
+      double *slot = slots + (size_t)(P.bin_start[b] / kCompGroupRecords) * (kNc * 64);
+#pragma unroll
+      for (int k = 0; k < kNc; ++k) {
+        const double x = n_in > 1 ? comb[k * 64 + lane] : (double)csum[k] + (double)ccmp[k];
+        if (x != 0.0) unsafeAtomicAdd(slot + k * 64 + lane, x);
+      }
+      return;
+    }
+  }
+  store_tile<R, NPOL, MB, VB>(P, acc, gplane, u0, v0, multi, accumulate);
+}
+
+// Compensated mode, around the gridder: clear the FP64 slots of split bins
+// (FINISH false), or round them to the grid (true).  A wavefront walks 64
+// units and takes the first unit of each split bin among them.
+template <int NPOL, int MB, int VB, bool FINISH>
+__global__ __launch_bounds__(256) void k_comp_slots(PlanDev P, float *grid, int accumulate) {
+  using MV = typename MfmaOp<float>::V;
+  constexpr int C = 2 * NPOL, kNc = MB * C * VB * 4;
+  double *slots = comp_slots(P, mfma_comb_bytes<NPOL, MB, VB, true>());
+  if (!slots) return;
+  const uint32_t n_units = P.gunit_start[P.n_bins];
+  const int lane = threadIdx.x & 63;
+  for (uint32_t w0 = (blockIdx.x * 4 + threadIdx.x / 64) * 64; w0 < n_units;
+       w0 += gridDim.x * 256) {
+    const uint4 mine = P.gunits[min(w0 + lane, n_units - 1)];
+    const uint32_t per = max(1u, kCompGroupRecords / (uint32_t)P.unit_cap);
+    const bool lead = w0 + lane < n_units && (mine.w & kUnitMulti) && (mine.w & kUnitFirst) &&
+                      P.gunit_start[mine.x + 1] - P.gunit_start[mine.x] > per;
+    for (unsigned long long m = __ballot(lead); m; m &= m - 1) {
+      const int64_t b = (uint32_t)__builtin_amdgcn_readlane((int)mine.x, __ffsll(m) - 1);
+      double *slot = slots + (size_t)(P.bin_start[b] / kCompGroupRecords) * (kNc * 64);
+      if constexpr (!FINISH) {
+#pragma unroll
+        for (int k = 0; k < kNc; ++k) slot[k * 64 + lane] = 0.0;
+      } else {
+        const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
+        const int ic = (int)((uint32_t)b - tile * (uint32_t)P.n_img_chan);
+        const uint32_t tu_i = tile / (uint32_t)P.ntv;
+        const int u0 = (int)tu_i * 16 * MB, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * 16 * VB;
+        MV acc[MB][C][VB];
+#pragma unroll
+        for (int k = 0; k < kNc; ++k)
+          acc[k / (C * VB * 4)][k / (VB * 4) % C][k / 4 % VB][k % 4] = (float)slot[k * 64 + lane];
+        store_tile<float, NPOL, MB, VB>(P, acc, grid + (size_t)ic * NPOL * P.n_u * P.n_v * 2, u0,
+                                        v0, false, accumulate != 0);
+      }
+    }
   }
 }
 
@@ -753,34 +909,45 @@ __global__ __launch_bounds__(256) void k_sumwt_reduce(PlanDev P, int npol, doubl
   }
 }
 
-// zero the tiles of bins that several units add into (overwrite mode): one
-// thread per unit reads the unit list in one coalesced pass; the thread of a
-// split bin's first unit clears that tile (such bins are few: those with more
-// records than a unit holds)
+// Before a tile kernel, in one launch: the call's tables (kTableBlocks
+// workgroups, when cgk is given) and, in overwrite mode (grid given), zeros
+// in the sums of weights and in the tiles of split bins, which several units
+// add into: a wavefront walks 64 units and clears the tile of each split
+// bin's first unit together.
 template <typename R>
-__global__ __launch_bounds__(256) void k_zero_multi(PlanDev P, R *grid, int npol) {
-  const uint32_t n_units = P.gunit_start[P.n_bins];
-  const int Tu = P.tile_u, Tv = P.tile_v;
-  for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < n_units;
-       u += gridDim.x * blockDim.x) {
-    const uint4 unit = P.gunits[u];
-    if (!((unit.w & kUnitMulti) && (unit.w & kUnitFirst))) continue;
-    const uint32_t tile = unit.x / (uint32_t)P.n_img_chan;
-    const int ic = (int)(unit.x - tile * (uint32_t)P.n_img_chan);
-    const uint32_t tu_i = tile / (uint32_t)P.ntv;
-    const int u0 = (int)tu_i * Tu, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * Tv;
-    const int u1 = min(u0 + Tu, P.n_u), v1 = min(v0 + Tv, P.n_v);
-    for (int p = 0; p < npol; ++p)
-      for (int gu = u0; gu < u1; ++gu) {
-        Cplx<R> *row = (Cplx<R> *)(grid + (((size_t)ic * npol + p) * P.n_u + gu) * P.n_v * 2);
-        for (int gv = v0; gv < v1; ++gv) row[gv] = Cplx<R>{(R)0, (R)0};
-      }
+__global__ __launch_bounds__(256) void k_grid_pre(PlanDev P, const double *cgk, R *grid, int npol,
+                                                  double *sumwt) {
+  const int tblocks = cgk ? kTableBlocks : 0;
+  if ((int)blockIdx.x < tblocks) {
+    fill_tables(P, cgk, blockIdx.x * blockDim.x + threadIdx.x, tblocks * blockDim.x);
+    return;
   }
-}
-
-__global__ void k_zero_f64(double *p, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
+  if (!grid) return;
+  const uint32_t blk = blockIdx.x - tblocks, nblk = gridDim.x - tblocks;
+  for (int64_t i = (int64_t)blk * blockDim.x + threadIdx.x; i < (int64_t)P.n_img_chan * npol;
+       i += (int64_t)nblk * blockDim.x)
+    sumwt[i] = 0.0;
+  const uint32_t n_units = P.gunit_start[P.n_bins];
+  const int Tu = P.tile_u, Tv = P.tile_v, lane = threadIdx.x & 63;
+  for (uint32_t w0 = (blk * 4 + threadIdx.x / 64) * 64; w0 < n_units; w0 += nblk * 256) {
+    const uint4 mine = P.gunits[min(w0 + lane, n_units - 1)];
+    const bool lead =
+        w0 + lane < n_units && (mine.w & kUnitMulti) && (mine.w & kUnitFirst);
+    for (unsigned long long m = __ballot(lead); m; m &= m - 1) {
+      const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)mine.x, __ffsll(m) - 1);
+      const uint32_t tile = b / (uint32_t)P.n_img_chan;
+      const int ic = (int)(b - tile * (uint32_t)P.n_img_chan);
+      const uint32_t tu_i = tile / (uint32_t)P.ntv;
+      const int u0 = (int)tu_i * Tu, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * Tv;
+      for (int p = 0; p < npol; ++p)
+        for (int c = lane; c < Tu * Tv; c += 64) {
+          const int gu = u0 + c / Tv, gv = v0 + c % Tv;
+          if (gu < P.n_u && gv < P.n_v)
+            *(Cplx<R> *)(grid + ((((size_t)ic * npol + p) * P.n_u + gu) * P.n_v + gv) * 2) =
+                Cplx<R>{(R)0, (R)0};
+        }
+    }
+  }
 }
 
 template <typename R, int NPOL, int DVW, bool COMP>
@@ -802,8 +969,6 @@ static int launch_grid(av_plan *plan, const void *vis, const void *weight, const
     const int rc_lds = ensure_lds_limit<k_grid_tiles<R, NPOL, DVW, COMP>>(L.total, "av_grid: hipFuncSetAttribute");
     if (rc_lds) return rc_lds;
   }
-  int rc = prepare_tables(d, cgk, s);
-  if (rc) return rc;
   // one wavefront per unit; the plan's capacity bounds the unit count
   const unsigned nwg = (unsigned)((d.max_gunits + nw - 1) / nw);
   hipLaunchKernelGGL(kfn, dim3(nwg), dim3(64 * nw), L.total, s, d,
@@ -826,17 +991,30 @@ static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
   const DeviceProps &prop = device_props();
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   const MfmaLds L = mfma_lds_layout<R, NPOL>(d.ov, d.support, 16 * (MB > VB ? MB : VB));
+  const int lds = L.total + mfma_comb_bytes<NPOL, MB, VB, COMP>();
   {
-    const int rc_lds = ensure_lds_limit<k_grid_mfma<R, NPOL, MB, VB, COMP, PSF>>(L.total, "av_grid: hipFuncSetAttribute");
+    const int rc_lds = ensure_lds_limit<k_grid_mfma<R, NPOL, MB, VB, COMP, PSF>>(lds, "av_grid: hipFuncSetAttribute");
     if (rc_lds) return rc_lds;
   }
-  int rc = prepare_tables(d, cgk, s);
-  if (rc) return rc;
-  const unsigned nwg = (unsigned)xcd_grouped_grid(
-      (d.max_gunits + kGridMaxWaves - 1) / kGridMaxWaves, kGridXcdGroup);
-  hipLaunchKernelGGL(kfn, dim3(nwg), dim3(kGridThreads), L.total, s, d, (const R *)vis,
+  const unsigned nsb = (unsigned)std::max<int64_t>(
+      1, std::min<int64_t>((d.max_gunits + 255) / 256, 4096));
+  if constexpr (COMP) {
+    hipLaunchKernelGGL((k_comp_slots<NPOL, MB, VB, false>), dim3(nsb), dim3(256), 0, s, d,
+                       (float *)grid, 0);
+    AV_LAUNCH_CHECK("k_comp_slots");
+  }
+  constexpr int kUnitsPerWg = COMP ? 1 : kGridMaxWaves;
+  const unsigned nwg =
+      (unsigned)xcd_grouped_grid((d.max_gunits + kUnitsPerWg - 1) / kUnitsPerWg,
+                                 kGridXcdGroup * kGridMaxWaves / kUnitsPerWg);
+  hipLaunchKernelGGL(kfn, dim3(nwg), dim3(kGridThreads), lds, s, d, (const R *)vis,
                      (const R *)weight, flag, cgk, (R *)grid, mode);
   AV_LAUNCH_CHECK("k_grid_mfma");
+  if constexpr (COMP) {
+    hipLaunchKernelGGL((k_comp_slots<NPOL, MB, VB, true>), dim3(nsb), dim3(256), 0, s, d,
+                       (float *)grid, mode & AV_GRID_ACCUMULATE);
+    AV_LAUNCH_CHECK("k_comp_slots");
+  }
   if (!(mode & AV_GRID_ADJOINT)) {
     hipLaunchKernelGGL(k_sumwt_reduce, dim3((unsigned)d.n_img_chan), dim3(256), 0, s, d, NPOL,
                        sumwt);
@@ -1195,8 +1373,6 @@ static int try_grid_h3(av_plan *plan, const void *vis, const void *weight, const
   const DeviceProps &prop = device_props();
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   if ((size_t)h3_lds_layout<NPOL>(d.ov, d.support).total > prop.lds_per_block) return AV_OK;
-  int rc = prepare_tables(d, cgk, s);
-  if (rc) return rc;
   done = true;
   if (mode & AV_GRID_PSF)
     return launch_grid_h3<NPOL, true>(plan, vis, weight, flag, grid, sumwt, mode, s);
@@ -1557,8 +1733,6 @@ static int try_grid_sub(av_plan *plan, const void *vis, const void *weight, cons
   const DeviceProps &prop = device_props();
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   if ((size_t)sub_lds_layout<NPOL>(d.ov, d.support).total > prop.lds_per_block) return AV_OK;
-  int rc = prepare_tables(d, cgk, s);
-  if (rc) return rc;
   done = true;
   if (mode & AV_GRID_PSF)
     return launch_grid_sub<NPOL, 1>(plan, vis, weight, flag, grid, sumwt, mode, s);
@@ -1586,7 +1760,8 @@ static int try_mfma(av_plan *plan, const void *vis, const void *weight, const ui
       if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
       const MfmaLds L = mfma_lds_layout<R, NPOL>(plan->d.ov, plan->d.support,
                                                  16 * (MB > VB ? MB : VB));
-      if ((size_t)L.total > prop.lds_per_block) return AV_OK;
+      if ((size_t)L.total + mfma_comb_bytes<NPOL, MB, VB, COMP>() > prop.lds_per_block)
+        return AV_OK;
       done = true;
       if (mode & AV_GRID_PSF)
         return launch_grid_mfma<R, NPOL, MB, VB, COMP, true>(plan, vis, weight, flag, cgk, grid,
@@ -1655,19 +1830,21 @@ static int dispatch_grid(av_plan *plan, const void *vis, const void *weight, con
   return launch_grid<R, NPOL, 16, false>(plan, vis, weight, flag, cgk, grid, sumwt, mode, s);
 }
 
-// Overwrite mode, before a tile kernel: zero the sums of weights and the
-// tiles of split bins (the units of a split bin add into them).
-int zero_before_grid(const PlanDev &d, void *grid, int npol, bool fp64, double *sumwt,
-                     hipStream_t s) {
-  int64_t n = (int64_t)d.n_img_chan * npol;
-  hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, sumwt, n);
-  AV_LAUNCH_CHECK("k_zero_f64");
-  const unsigned zb = (unsigned)std::min<int64_t>((d.max_gunits + 255) / 256, 8192);
+// Before a tile kernel: the call's tables (cgk given) and, in overwrite mode
+// (grid given), zeros in the sums of weights and in the tiles of split bins.
+int prepare_grid(const PlanDev &d, const double *cgk, void *grid, int npol, bool fp64,
+                 double *sumwt, hipStream_t s) {
+  const unsigned zb =
+      (unsigned)((cgk ? kTableBlocks : 0) +
+                 (grid ? std::min<int64_t>((d.max_gunits + 255) / 256, 4096) : 0));
+  if (zb == 0) return AV_OK;
   if (fp64)
-    hipLaunchKernelGGL(k_zero_multi<double>, dim3(zb), dim3(256), 0, s, d, (double *)grid, npol);
+    hipLaunchKernelGGL(k_grid_pre<double>, dim3(zb), dim3(256), 0, s, d, cgk, (double *)grid, npol,
+                       sumwt);
   else
-    hipLaunchKernelGGL(k_zero_multi<float>, dim3(zb), dim3(256), 0, s, d, (float *)grid, npol);
-  AV_LAUNCH_CHECK("k_zero_multi");
+    hipLaunchKernelGGL(k_grid_pre<float>, dim3(zb), dim3(256), 0, s, d, cgk, (float *)grid, npol,
+                       sumwt);
+  AV_LAUNCH_CHECK("k_grid_pre");
   return AV_OK;
 }
 
@@ -1684,10 +1861,9 @@ static int grid_by_pol(av_plan *plan, const void *vis, const void *weight, const
                        int npol, const double *cgk, void *grid, double *sumwt, int mode,
                        hipStream_t s) {
   PlanDev &d = plan->d;
-  if (!(mode & AV_GRID_ACCUMULATE)) {
-    const int rc = zero_before_grid(d, grid, npol, sizeof(R) == 8, sumwt, s);
-    if (rc) return rc;
-  }
+  const int rc = prepare_grid(d, cgk, (mode & AV_GRID_ACCUMULATE) ? nullptr : grid, npol,
+                              sizeof(R) == 8, sumwt, s);
+  if (rc) return rc;
   switch (npol) {
     case 1: return dispatch_grid<R, 1>(plan, vis, weight, flag, cgk, grid, sumwt, mode, s);
     case 2: return dispatch_grid<R, 2>(plan, vis, weight, flag, cgk, grid, sumwt, mode, s);

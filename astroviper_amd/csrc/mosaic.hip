@@ -310,7 +310,7 @@ static int launch_mosaic(av_plan *plan, MosaicArgs<R> A, double *sumwt, int mode
   }
   const bool accumulate = (mode & AV_GRID_ACCUMULATE) != 0;
   if (!accumulate) {
-    const int rc = zero_before_grid(d, A.grid, NPOL, sizeof(R) == 8, sumwt, s);
+    const int rc = prepare_grid(d, nullptr, A.grid, NPOL, sizeof(R) == 8, sumwt, s);
     if (rc) return rc;
   }
   // the kernel-sum table, in stream-ordered memory freed after the gridder

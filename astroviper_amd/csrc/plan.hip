@@ -21,7 +21,7 @@
 // every row carries its own channel).
 #include <algorithm>
 
-#include "avgrid_internal.h"
+#include "tile_common.h"
 
 namespace av {
 
@@ -953,44 +953,12 @@ static int launch_index(const PlanDev &d, hipStream_t s) {
   return AV_OK;
 }
 
-// per-call tables: the FP32 kernel table; for every kernel offset, the FP64
-// sum of the support taps of one axis (norm = nrm[ou] * nrm[ov]); and the
-// zero-padded weight table by (tap, offset) in FP32 and FP64.  Offsets past
-// ov/2 (never produced by a sample) read 0 beyond the end of the table.
 __global__ void k_prepare_tables(PlanDev P, const double *cgk) {
-  const int sc = P.support / 2, ov = P.ov;
-  const int ntab = ov * (sc + 1), half = ov / 2 + 2, nnrm = 2 * half + 1;
-  const int nw = (P.support + 2) * nnrm;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ntab + nnrm + nw;
-       i += gridDim.x * blockDim.x) {
-    if (i < ntab) {
-      P.tab32[i] = (float)cgk[i];
-    } else if (i < ntab + nnrm) {
-      const int off = i - ntab - half;
-      double s = 0.0;
-      for (int t = 0; t < P.support; ++t) {
-        int k = ov * (t - sc) + off;
-        k = k < 0 ? -k : k;
-        s += k < ntab ? cgk[k] : 0.0;
-      }
-      P.nrm[i - ntab] = s;
-    } else {
-      const int j = i - ntab - nnrm;
-      const int tc = j / nnrm - 1, off = j - (j / nnrm) * nnrm - half;
-      double v = 0.0;
-      if (tc >= 0 && tc < P.support) {
-        int k = ov * (tc - sc) + off;
-        k = k < 0 ? -k : k;
-        v = k < ntab ? cgk[k] : 0.0;
-      }
-      P.wtab32[j] = (float)v;
-      P.wtab64[j] = v;
-    }
-  }
+  fill_tables(P, cgk, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 int prepare_tables(const PlanDev &d, const double *cgk, hipStream_t s) {
-  hipLaunchKernelGGL(k_prepare_tables, dim3(4), dim3(256), 0, s, d, cgk);
+  hipLaunchKernelGGL(k_prepare_tables, dim3(kTableBlocks), dim3(256), 0, s, d, cgk);
   AV_LAUNCH_CHECK("k_prepare_tables");
   return AV_OK;
 }
@@ -1009,6 +977,20 @@ __global__ void k_popcount(const unsigned long long *m, int64_t n, uint32_t *out
 using namespace av;
 
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Records per work unit when the caller leaves it open.  A unit is one
+// wavefront's serial walk over its records, so a plan of few samples needs
+// short units to spread its dense central bins over the chip, and a plan of
+// many samples long ones, since the tiles of a split bin are added with
+// atomics.  Measured (bin + grid + degrid, us) at caps of 8192, 2048, 1024,
+// 512, 256 and 128: 28,080 samples FP64 297, 294, 246, 188, 162, 160; 4.8 M
+// FP64 2364, 2340, 2227, 2272, 2320, 2725; 35 M FP32 6586, 6113, 6249, 6639,
+// 7889, 12779.
+static int32_t default_unit_cap(int64_t n_items) {
+  int32_t cap = 256;
+  while (cap < 8192 && (int64_t)cap * kCapSamples * 3 < n_items * 2) cap *= 2;
+  return cap;
+}
 
 // Rows of a chunk.  Every chunk is a workgroup of the two binning passes:
 // kChunkTarget of them in all keep the chip busy, but a chunk also reads and
@@ -1035,7 +1017,8 @@ static int32_t chunk_rows(int64_t n_rows, int32_t n_chan, int64_t ntiles, bool a
 // of device memory the plan's arrays need; with base non-NULL, also point
 // the arrays into [base, base + bytes).  Shared by av_plan_create (one
 // hipMalloc) and av_grid_noalloc (the library's static scratch array).  With
-// `compact`, chunks are as long as they may be: the fewest bytes.
+// `compact`, chunks and default units are as long as they may be: the fewest
+// bytes.
 int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u, int32_t n_v,
                 double cell_u, double cell_v, int32_t support, int32_t oversampling,
                 int32_t tile_u, int32_t tile_v, int32_t geometry, int32_t unit_cap, av_plan *p,
@@ -1063,7 +1046,7 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   if (conjugate && geometry != AV_GEOM_REFERENCE)
     return fail(AV_ERR_INVALID, "av_plan_create: AV_GEOM_CONJUGATE needs AV_GEOM_REFERENCE");
   int64_t n_items = row_channels ? n_rows : n_rows * (int64_t)n_chan;
-  if (unit_cap == 0) unit_cap = 8192;
+  if (unit_cap == 0) unit_cap = compact ? 8192 : default_unit_cap(n_items);
   if (unit_cap < 64) return fail(AV_ERR_INVALID, "av_plan_create: unit_cap < 64");
   if (n_items > ((int64_t)1 << 32) / 5 - 1)
     return fail(AV_ERR_UNSUPPORTED, "av_plan_create: more than 858993458 samples per plan");

@@ -216,4 +216,41 @@ __device__ inline void h3_split_products8(const float *w, const float *d, H3U4 &
   lo = H3U4{l0, l1, l2, l3};
 }
 
+// per-call tables: the FP32 kernel table; for every kernel offset, the FP64
+// sum of the support taps of one axis (norm = nrm[ou] * nrm[ov]); and the
+// zero-padded weight table by (tap, offset) in FP32 and FP64.  Offsets past
+// ov/2 (never produced by a sample) read 0 beyond the end of the table.
+// Thread `id` of `n`.
+constexpr int kTableBlocks = 4;  // workgroups of 256 threads that share the work
+__device__ inline void fill_tables(const PlanDev &P, const double *cgk, int id, int n) {
+  const int sc = P.support / 2, ov = P.ov;
+  const int ntab = ov * (sc + 1), half = ov / 2 + 2, nnrm = 2 * half + 1;
+  const int nw = (P.support + 2) * nnrm;
+  for (int i = id; i < ntab + nnrm + nw; i += n) {
+    if (i < ntab) {
+      P.tab32[i] = (float)cgk[i];
+    } else if (i < ntab + nnrm) {
+      const int off = i - ntab - half;
+      double s = 0.0;
+      for (int t = 0; t < P.support; ++t) {
+        int k = ov * (t - sc) + off;
+        k = k < 0 ? -k : k;
+        s += k < ntab ? cgk[k] : 0.0;
+      }
+      P.nrm[i - ntab] = s;
+    } else {
+      const int j = i - ntab - nnrm;
+      const int tc = j / nnrm - 1, off = j - (j / nnrm) * nnrm - half;
+      double v = 0.0;
+      if (tc >= 0 && tc < P.support) {
+        int k = ov * (tc - sc) + off;
+        k = k < 0 ? -k : k;
+        v = k < ntab ? cgk[k] : 0.0;
+      }
+      P.wtab32[j] = (float)v;
+      P.wtab64[j] = v;
+    }
+  }
+}
+
 }  // namespace av

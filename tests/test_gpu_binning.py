@@ -76,3 +76,35 @@ def test_binning_paths_match_oracle(gpu, oracle, nt, nb, nchan, n_u, n_v, cube):
             assert _rel(sw, swref) < 1e-12
             assert _rel(m.reshape(mref.shape), mref) < 1e-12
         assert st["grid_units"] >= st["bins"]
+
+
+@pytest.mark.parametrize("cap", [64, 1024, 8192, 0])
+@pytest.mark.parametrize("tile", [(16, 16), (32, 32), (24, 24)])
+def test_compensated_sums_of_split_bins(gpu, oracle, cap, tile):
+    """Compensated sums of bins of far more records than a unit holds (about
+    20,000 per central tile) against the oracle.  Weights of one sign: a
+    term's rounding (sample and table in FP32, one product each) stays below
+    4 * 2^-24 of it, and 20,000 / 8192 groups add at most three roundings of
+    the sum, so 8 * 2^-24 = 4.8e-7 of the largest cell bounds the error."""
+    from astroviper_amd.device import GridPlan
+    n_uv = (64, 64)
+    nt, nb, nchan, npol = 120, 500, 2, 1
+    uvw, freq, _, w, flag, cell = _samples(nt, nb, nchan, npol, n_uv, 5, spread=0.3)
+    w = w.astype(np.float32)
+    gref, swref = oracle.standard_grid(None, uvw, np.where(flag, 0, w).astype(float), freq, n_uv,
+                                       cell, chan_mode="continuum", do_psf=True)
+    rows = nt * nb
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(rows, nchan, 1, n_uv, cell, tile=tile, unit_cap=cap, device=gpu)
+    plan.set_uvw(dev(uvw.reshape(rows, 3)), dev(freq))
+    g, sw = plan.grid(None, dev(w.reshape(-1, npol)),
+                      dev(flag.reshape(-1, npol).astype(np.uint8)), psf=True, compensated=True)
+    assert _rel(g.cpu().numpy(), gref) < 8 * 2.0 ** -24
+    assert _rel(sw.cpu().numpy(), swref) < 1e-12
+    # accumulating the same samples doubles the grid
+    g2, sw2 = plan.grid(None, dev(w.reshape(-1, npol)),
+                        dev(flag.reshape(-1, npol).astype(np.uint8)), grid=g, sumwt=sw, psf=True,
+                        accumulate=True, compensated=True)
+    assert _rel(g2.cpu().numpy(), 2 * gref) < 16 * 2.0 ** -24
+    assert _rel(sw2.cpu().numpy(), 2 * swref) < 1e-12
+    plan.close()
