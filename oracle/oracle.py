@@ -378,7 +378,10 @@ def hogbom_clean(dirty_image, psf, mask=None, clean_box=(-1, -1, -1, -1), max_it
     """clean (hclean.cpp:106-210 through bindings.cpp:61-193, no callbacks):
     the result dictionary of the reference's extension."""
     d = np.ascontiguousarray(dirty_image)
-    dt = np.float32 if d.dtype == np.float32 else np.float64
+    # the overload the extension picks (bindings.cpp:243-301): float64 only
+    # when every array given is float64, an empty mask included
+    given = [d, np.asarray(psf)] + ([] if mask is None else [np.asarray(mask)])
+    dt = np.float64 if all(a.dtype == np.float64 for a in given) else np.float32
     resid = d.astype(dt, copy=True)
     p = np.ascontiguousarray(psf, dtype=dt)
     ny, nx = resid.shape
