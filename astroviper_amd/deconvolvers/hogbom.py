@@ -177,6 +177,35 @@ def clean_device(residual: torch.Tensor, psf: torch.Tensor, model: torch.Tensor,
     return it
 
 
+def clean_planes_device(residual: torch.Tensor, psf: torch.Tensor, model: torch.Tensor,
+                        planes_per_psf: int, max_iter: int, gain: float = 0.1,
+                        threshold: float = 0.0, work: Optional[torch.Tensor] = None):
+    """CLEAN planes [n, ny, nx] in place, as :func:`clean_device` each from
+    iteration 0 over its whole extent, side by side on the chip: plane p with
+    psf[p // planes_per_psf].  Device tensors of one dtype, float32 or
+    float64.  Returns the iterations of each plane (NumPy int32 [n])."""
+    n, ny, nx = residual.shape
+    for t in (residual, psf, model):
+        if t.dtype != residual.dtype or tuple(t.shape[1:]) != (ny, nx) or not t.is_contiguous():
+            raise ValueError("residual, psf and model must be contiguous [planes, ny, nx] "
+                             "tensors of one dtype")
+    if model.shape[0] != n or psf.shape[0] * planes_per_psf < n:
+        raise ValueError("every residual plane needs a model plane and a PSF")
+    if max_iter > (1 << 32) // 1024 - 2:
+        raise ValueError("too many iterations for one call")
+    dt = np.float32 if residual.dtype == torch.float32 else np.float64
+    if work is None:
+        work = _work(residual.device)
+    result = torch.empty((n, 6), dtype=torch.int32, device=residual.device)
+    _lib.call("av_hogbom_clean_planes", _dev._ptr(model), _dev._ptr(residual), _dev._ptr(psf), n,
+              int(planes_per_psf), nx, ny, int(max_iter), float(dt(gain)), float(dt(threshold)),
+              _code(dt), _dev._ptr(result), _dev._ptr(work), _dev._stream())
+    head = result.cpu().numpy()
+    if np.any(head[:, 3] < 0):
+        raise _lib.AvgridError("av_hogbom_clean_planes: a workgroup did not reach the exchange")
+    return head[:, 0]
+
+
 def clean(dirty_image, psf, mask=None, clean_box=(-1, -1, -1, -1), max_iter: int = 100,
           start_iter: int = 0, gain: float = 0.1, threshold: float = 0.0, speedup: float = 0.0,
           progress_callback=None, stop_callback=None) -> dict:

@@ -167,18 +167,21 @@ class ResidentImager:
         nch, npol = dirty.shape[:2]
         if self._work is None:
             self._work = H._work(self.dev)
-        comps = torch.zeros(dirty.shape, dtype=torch.float64, device=self.dev)
+        comps = torch.empty(dirty.shape, dtype=torch.float64, device=self.dev)
         resid = torch.empty(dirty.shape, dtype=torch.float64, device=self.dev)
         iters = np.zeros((nch, npol), dtype=np.int64)
-        for c in range(nch):
-            p = psf[c, 0].to(clean_dtype).contiguous()
-            for q in range(npol):
-                r = dirty[c, q].to(clean_dtype).contiguous()
-                m = torch.zeros_like(r)
-                iters[c, q] = H.clean_device(r, p, m, None, None, int(niter), 0, gain, threshold,
-                                             work=self._work)
-                comps[c, q] = m.to(torch.float64)
-                resid[c, q] = r.to(torch.float64)
+        # channels per call: the planes run side by side, in copies of at most
+        # about 2 GiB
+        step = max(1, (1 << 28) // max(1, npol * self.ny * self.nx))
+        for c0 in range(0, nch, step):
+            c1 = min(nch, c0 + step)
+            r = dirty[c0:c1].reshape((-1,) + tuple(dirty.shape[2:])).to(clean_dtype, copy=True)
+            p = psf[c0:c1, 0].to(clean_dtype).contiguous()
+            m = torch.zeros_like(r)
+            iters[c0:c1] = H.clean_planes_device(r, p, m, npol, int(niter), gain, threshold,
+                                                 work=self._work).reshape(c1 - c0, npol)
+            comps[c0:c1] = m.reshape(dirty[c0:c1].shape)
+            resid[c0:c1] = r.reshape(dirty[c0:c1].shape)
         return comps, resid, iters
 
     def write_back(self, ms4) -> None:

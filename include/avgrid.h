@@ -65,7 +65,7 @@ extern "C" {
 
 /* ABI version: bumped whenever a signature changes; the bindings refuse a
  * library whose version differs from the one they were written for. */
-#define AV_ABI_VERSION 12
+#define AV_ABI_VERSION 13
 
 const char *av_last_error(void);
 int av_version(void);
@@ -345,6 +345,18 @@ int av_hogbom_clean(void *model, void *residual, const void *psf,
                     int32_t skip_report, double gain, double thres,
                     double cspeedup, int32_t px0, int32_t py0, int32_t dtype,
                     void *work, void *stream);
+
+/* clean of n_planes planes in one call, each from iteration 0 over its whole
+ * extent, no mask, callbacks or speed-up: the plane loop of
+ * deconvolution.py:224-287.  model and residual [n_planes][ny][nx]; plane p
+ * uses PSF p / planes_per_psf of psf [..][ny][nx].  result: n_planes records
+ * of 24 bytes {int32 iterations, x, y of the last peak, reason; double last
+ * peak}; reason -1 says that a workgroup did not reach an exchange.  Planes
+ * run side by side on the chip. */
+int av_hogbom_clean_planes(void *model, void *residual, const void *psf, int32_t n_planes,
+                           int32_t planes_per_psf, int32_t nx, int32_t ny, int32_t niter,
+                           double gain, double thres, int32_t dtype, void *result, void *work,
+                           void *stream);
 
 /* ---------------------------------------------------- imaging weights --
  * core/imaging/imaging_weighting/grid_imaging_weights.py.  uvw [n_rows][3]
