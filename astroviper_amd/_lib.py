@@ -11,7 +11,7 @@ import os
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libavgrid.so")
 
-AV_ABI_VERSION = 13  # must equal AV_ABI_VERSION of include/avgrid.h
+AV_ABI_VERSION = 14  # must equal AV_ABI_VERSION of include/avgrid.h
 
 AV_OK = 0
 AV_ERR_INVALID = -1
@@ -77,6 +77,9 @@ SIGNATURES = {
     "av_ifftshift_hermitian": (_c.c_int, [_P, _P, _I64, _I32, _I32, _I32, _P]),
     "av_normalise_real": (_c.c_int, [_P, _P, _P, _P, _I64, _I32, _I32, _P, _I32, _P]),
     "av_hermitian_expand": (_c.c_int, [_P, _P, _I64, _I32, _I32, _I32, _I32, _P]),
+    "av_fft_work_bytes": (_c.c_int, [_I64, _I32, _I32, _P]),
+    "av_uv_to_image": (_c.c_int, [_P, _I32, _I64, _I32, _I32, _P, _I32, _P, _I32, _P, _P]),
+    "av_image_to_uv": (_c.c_int, [_P, _I32, _I64, _I32, _I32, _I32, _P, _I32, _P, _P]),
     "av_hogbom_work_bytes": (_c.c_int, [_P]),
     "av_hogbom_maximg": (_c.c_int, [_P, _P, _I32, _I32, _I32, _P, _P]),
     "av_hogbom_clean": (_c.c_int, [_P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32,

@@ -349,6 +349,37 @@ def degrid_kernel_name(tile, n_pol: int, support: int = 7, fp64: bool = False,
     return "k_degrid_mfma" if blocks <= 16 else "k_degrid_tiles"
 
 
+# ---------------------------------------------------------------- FFTs --
+def fft_work(planes: int, n_u: int, n_v: int, device) -> Optional[torch.Tensor]:
+    """Work memory for uv_to_image / image_to_uv on planes of n_u x n_v; None
+    for sizes they do not serve (odd axes, prime factors beyond 5, very long
+    ones)."""
+    n = ctypes.c_int64()
+    call("av_fft_work_bytes", int(planes), int(n_u), int(n_v), ctypes.byref(n))
+    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
+
+
+def uv_to_image(grid: torch.Tensor, sumwt: Optional[torch.Tensor], out: torch.Tensor,
+                work: torch.Tensor, taper: bool = True) -> torch.Tensor:
+    """real(fftshift(N^2 ifft2(ifftshift(grid)))) / taper / sumwt per plane
+    into `out` (real), in FP64."""
+    n_u, n_v = grid.shape[-2:]
+    call("av_uv_to_image", _ptr(_aligned(grid, 16)), _real_code(grid.dtype),
+         grid.numel() // (n_u * n_v), n_u, n_v, _ptr(sumwt), int(taper), _ptr(out),
+         _real_code(out.dtype), _ptr(work), _stream())
+    return out
+
+
+def image_to_uv(image: torch.Tensor, out: torch.Tensor, work: torch.Tensor,
+                taper: bool = False) -> torch.Tensor:
+    """fftshift(fft2(ifftshift(image / taper))) of a real image into `out`
+    (complex), in FP64."""
+    n_u, n_v = image.shape[-2:]
+    call("av_image_to_uv", _ptr(_aligned(image, 16)), _real_code(image.dtype),
+         image.numel() // (n_u * n_v), n_u, n_v, int(taper), _ptr(out), _real_code(out.dtype), _ptr(work), _stream())
+    return out
+
+
 # --------------------------------------------------------- dirty image --
 def dirty_image(grid: torch.Tensor, sumwt: torch.Tensor, support: int = 7,
                 oversampling: int = 100, out_dtype: torch.dtype = torch.float64,
@@ -363,19 +394,25 @@ def dirty_image(grid: torch.Tensor, sumwt: torch.Tensor, support: int = 7,
 
     FP64 transforms of even-sized planes go through a complex-to-real FFT:
     only the real part of the inverse FFT is kept, and it is the transform of
-    the grid's Hermitian half spectrum, which av_ifftshift_hermitian folds
-    (with both shifts) in one pass; the FFT then does half the work and the
-    passes around it move half the bytes.  Other cases transform the whole
-    complex planes (`work`, if given, holds them).
+    the grid's Hermitian half spectrum.  Axes without prime factors beyond 5
+    take av_uv_to_image, two passes that do everything; other even ones fold
+    the half spectrum (av_ifftshift_hermitian), transform it with torch.fft
+    and normalise.  Other cases transform the whole complex planes (`work`,
+    if given, holds them).
     """
     code = _real_code(grid.dtype)
     fcode = _real_code(fft_dtype)
     n_u, n_v = grid.shape[-2:]
     planes = grid.numel() // (n_u * n_v)
     g = grid.contiguous()
+    sw = sumwt.contiguous().to(torch.float64)
+    if fft_dtype == torch.complex128:
+        scratch = fft_work(planes, n_u, n_v, g.device)
+        if scratch is not None:
+            out = torch.empty(grid.shape, dtype=out_dtype, device=grid.device)
+            return uv_to_image(g, sw, out, scratch)
     tu = ps_correction_1d(n_u, grid.device)
     tv = tu if n_v == n_u else ps_correction_1d(n_v, grid.device)
-    sw = sumwt.contiguous().to(torch.float64)
     if fft_dtype == torch.complex128 and n_u % 2 == 0 and n_v % 2 == 0:
         half = torch.empty(g.shape[:-1] + (n_v // 2 + 1,), dtype=torch.complex128,
                            device=g.device)

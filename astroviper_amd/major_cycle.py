@@ -48,12 +48,20 @@ def model_to_uv(model: torch.Tensor, cdt: torch.dtype) -> torch.Tensor:
     place: two passes of the cube instead of the four of two rolls.
 
     A real image (the model) goes through a real-to-complex FFT, which
-    computes half the spectrum for half the work: the flipped image is
-    formed in the real dtype in one pass, transformed, and
-    av_hermitian_expand writes the whole spectrum from the half
+    computes half the spectrum for half the work.  In FP64, even axes without
+    prime factors beyond 5 take av_image_to_uv, two passes that do everything;
+    else the flipped image is formed in the real dtype in one pass, transformed,
+    and av_hermitian_expand writes the whole spectrum from the half
     (F[-k] = conj(F[k])) with the output flip, in one pass."""
     ny, nx = model.shape[-2:]
     ax = (-2, -1)
+    if not model.is_complex() and cdt == torch.complex128:
+        work = D.fft_work(model.numel() // max(1, ny * nx), ny, nx, model.device)
+        if work is not None:
+            if model.dtype not in (torch.float32, torch.float64):
+                model = model.to(torch.float64)
+            y = torch.empty(model.shape, dtype=cdt, device=model.device)
+            return D.image_to_uv(model.contiguous(), y, work)
     if ny % 4 or nx % 4:
         m = model.to(cdt)
         return torch.fft.fftshift(torch.fft.fft2(torch.fft.ifftshift(m, dim=ax), dim=ax), dim=ax)

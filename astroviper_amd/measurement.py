@@ -63,12 +63,23 @@ class MeasurementOperator:
              shift_u, shift_v, _dev._ptr(self.tu), _dev._ptr(self.tv), taper, float(scale),
              src_code, int(src_real), dst_code, int(dst_real), _dev._stream())
 
+    def _work(self):
+        """Work memory of the fused real FFTs, or None where they do not
+        serve the image size."""
+        return _dev.fft_work(self.n_img_chan * self.n_pol, self.n_u, self.n_v, self.device)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """Model visibilities [samples, n_pol] of image x (real or complex)."""
         x = x.reshape(self.shape).contiguous()
         real = not x.is_complex()
         rdt = _dev.real_dtype(self.code)
         x = x.to(rdt if real else self.cdtype)
+        if real:
+            work = self._work()
+            if work is not None:
+                g = torch.empty(self.shape, dtype=self.cdtype, device=self.device)
+                _dev.image_to_uv(x, g, work, taper=True)
+                return self.plan.degrid(g, n_pol=self.n_pol)
         w = torch.empty(self.shape, dtype=self.fft_dtype, device=self.device)
         # ifftshift, dividing by the taper at the source pixel
         self._pass(x, w, self.n_u // 2, self.n_v // 2, 1, 1.0, real, False, self.code,
@@ -84,6 +95,12 @@ class MeasurementOperator:
         y = y.reshape(self.n_samples, self.n_pol).to(self.cdtype).contiguous()
         g, _ = self.plan.grid(y, None, adjoint=True, n_pol=self.n_pol,
                               compensated=self.compensated)
+        if real:
+            work = self._work()
+            if work is not None:
+                out = torch.empty(self.shape, dtype=_dev.real_dtype(self.code),
+                                  device=self.device)
+                return _dev.uv_to_image(g, None, out, work)
         w = torch.empty(self.shape, dtype=self.fft_dtype, device=self.device)
         self._pass(g, w, self.n_u // 2, self.n_v // 2, 0, 1.0, False, False, self.code,
                    self.fcode)

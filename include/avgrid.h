@@ -65,7 +65,7 @@ extern "C" {
 
 /* ABI version: bumped whenever a signature changes; the bindings refuse a
  * library whose version differs from the one they were written for. */
-#define AV_ABI_VERSION 13
+#define AV_ABI_VERSION 14
 
 const char *av_last_error(void);
 int av_version(void);
@@ -309,6 +309,23 @@ int av_normalise_real(const double *image, const double *sumwt,
 int av_hermitian_expand(const void *half, void *out, int64_t n_planes,
                         int32_t n_u, int32_t n_v, int32_t sign, int32_t dtype,
                         void *stream);
+
+/* The whole image step of grid2image_spheroid_ms4 (standard_grid.py:693-708)
+ * for a real image: real(fftshift(N^2 ifft2(ifftshift(grid)))), over the
+ * taper (the outer product of grdsf on both axes) when `taper`, over
+ * sumwt [n_planes] when not NULL, in FP64.  And its counterpart
+ * fftshift(fft2(ifftshift(image / taper))) of a real image (fft_lm_to_uv,
+ * core/imaging/fft.py:5-18), in FP64 too.  Axes must be even with no prime
+ * factor beyond 5, n_u <= 4096 and n_v <= 16384: av_fft_work_bytes gives the
+ * bytes of `work` a call needs, 0 for other sizes.  Arrays start on 16-byte
+ * boundaries. */
+int av_fft_work_bytes(int64_t n_planes, int32_t n_u, int32_t n_v, int64_t *bytes);
+int av_uv_to_image(const void *grid, int32_t dtype, int64_t n_planes, int32_t n_u, int32_t n_v,
+                   const double *sumwt, int32_t taper, void *image, int32_t image_dtype,
+                   void *work, void *stream);
+int av_image_to_uv(const void *image, int32_t image_dtype, int64_t n_planes, int32_t n_u,
+                   int32_t n_v, int32_t taper, void *grid, int32_t dtype, void *work,
+                   void *stream);
 
 /* ------------------------------------------------------- Hogbom CLEAN --
  * core/imaging/deconvolvers/hogbom (the _hogbom_ext extension).  Images are
