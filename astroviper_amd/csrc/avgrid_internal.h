@@ -44,7 +44,7 @@ constexpr int kMaxRowsPerChunk = 124 * kChunkThreads;  // rows of one chunked-bi
 constexpr int64_t kChunkTarget = 1024;  // chunks a plan is cut into when its rows allow
 constexpr int kChunkAllChans = 2;       // channels of a continuum plan whose chunks span them all
 constexpr int64_t kCapSamples = 12288;  // samples of a plan per record of its default unit cap
-constexpr int kRowBlockRows = 8 * kChunkThreads;  // rows of a row-block binning workgroup
+constexpr int kMaxRowBlockRows = 16 * kChunkThreads;  // rows of a row-block binning workgroup
 
 // Packed geometry of one sample relative to a tile origin:
 // bits 0-7 u position + 16, 8-15 u offset + 128, 16-23 v position + 16,
@@ -164,6 +164,10 @@ struct PlanDev {
   int32_t row_channels;  // every row is one sample at its own channel
   int32_t ntu, ntv;      // tiles per axis
   int64_t n_bins;        // ntu * ntv * n_img_chan
+  // bins are numbered tile by tile, image channel by image channel within a
+  // tile, or (chan_major, rows that carry their own channel) the other way
+  int32_t chan_major;
+  uint32_t bin_minor;    // n_img_chan, or ntu * ntv when chan_major
   int64_t n_items;       // samples (row, chan)
   int64_t max_records;   // capacity of the record arrays
   int64_t max_gunits, max_dunits;
@@ -186,7 +190,7 @@ struct PlanDev {
   uint4 *gunits, *dunits;
   // pair units of the split-FP16 degridder (16 x 16 tiles, support <= 7):
   // tiles 2j and 2j + 1 along v of one image channel share a unit, pair p =
-  // (tile row, j, image channel) channel-minor; a unit is {bin of tile 2j,
+  // (tile row, j, image channel), channel-minor or -major as the bins; a unit is {bin of tile 2j,
   // first index into the pair's primary records (those of tile 2j, then
   // those of tile 2j + 1), count, bin of tile 2j + 1 or kNoBin}
   int64_t n_pairs, max_punits;      // 0 when the plan has no pair units
@@ -208,10 +212,10 @@ struct PlanDev {
   uint32_t *chunk_dup;              // [chunk][ntu * ntv]
   int32_t chunk_scatter;            // records written through per-chunk LDS cursors
   int32_t order_nb;                 // baselines per time step of time-major rows (1: row order)
-  // row-block binning (rows carry their own channel): kRowBlockRows rows per
+  // row-block binning (rows carry their own channel): row_block_rows rows per
   // workgroup, per-tile counters and cursors in LDS; the counting pass keeps
   // each block's own-channel counts (prim | dup << 16) for the scatter pass
-  int32_t row_blocks;
+  int32_t row_blocks, row_block_rows;
   uint32_t *row_hist;               // [row blocks][ntu * ntv], or NULL
   // per-call tables: FP32 kernel table, FP64 per-axis kernel sums by offset
   float *tab32;                     // [ov * (support/2 + 1)]
@@ -222,6 +226,18 @@ struct PlanDev {
   double *upart;                    // [max_gunits * 4]
   uint32_t *counters;               // scratch for statistics
 };
+
+// The number of tile `tile`'s bin of image channel ic, and back.
+__device__ inline int64_t bin_number(const PlanDev &P, int64_t tile, int ic) {
+  return P.chan_major ? (int64_t)ic * P.bin_minor + tile : tile * P.bin_minor + ic;
+}
+__device__ inline void bin_parts(const PlanDev &P, uint32_t b, uint32_t &tile, int &ic) {
+  // 32-bit divisions: bins are numbered below 2^32 (64-bit ones cost about a
+  // hundred scalar instructions each)
+  const uint32_t q = b / P.bin_minor, r = b - q * P.bin_minor;
+  tile = P.chan_major ? r : q;
+  ic = (int)(P.chan_major ? q : r);
+}
 
 constexpr uint32_t kNoBin = 0xFFFFFFFFu;  // a pair unit's missing second tile
 constexpr uint32_t kUnitMulti = 1u;  // bin split over several units

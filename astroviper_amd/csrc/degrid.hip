@@ -151,10 +151,9 @@ __global__ __launch_bounds__(kDegridThreads) void k_degrid_tiles(
   const uint4 unit = P.dunits[u];
   const int64_t b = unit.x;
   const uint32_t first = unit.y, cnt = unit.z;
-  // 32-bit divisions: bins are numbered below 2^32 (64-bit ones cost
-  // about a hundred scalar instructions each)
-  const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
-  const int ic = (int)((uint32_t)b - tile * (uint32_t)P.n_img_chan);
+  uint32_t tile;
+  int ic;
+  bin_parts(P, (uint32_t)b, tile, ic);
   const uint32_t tu_i = tile / (uint32_t)P.ntv;
   const int u0 = (int)tu_i * Tu, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * Tv;
   const R *gplane = grid + (size_t)ic * npol_g * P.n_u * P.n_v * 2;
@@ -484,10 +483,9 @@ void k_degrid_mfma(
 
   const WTab W(ov, S);
   copy_wtab(tab, W, P);
-  // 32-bit divisions: bins are numbered below 2^32 (64-bit ones cost
-  // about a hundred scalar instructions each)
-  const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
-  const int ic = (int)((uint32_t)b - tile * (uint32_t)P.n_img_chan);
+  uint32_t tile;
+  int ic;
+  bin_parts(P, (uint32_t)b, tile, ic);
   const uint32_t tu_i = tile / (uint32_t)P.ntv;
   const int u0 = (int)tu_i * Tu, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * Tv;
   const R *gplane = grid + (size_t)ic * npol_g * P.n_u * P.n_v * 2;
@@ -919,8 +917,9 @@ void k_degrid_h3(PlanDev P, const float *__restrict__ grid, int npol_g,
     const int n = W.size();
     for (int i = tid; i < n; i += kDegridThreads) tab[i] = P.wtab32[i] * 16384.0f;
   }
-  const uint32_t tile = (uint32_t)b / (uint32_t)P.n_img_chan;
-  const int ic = (int)((uint32_t)b - tile * (uint32_t)P.n_img_chan);
+  uint32_t tile;
+  int ic;
+  bin_parts(P, (uint32_t)b, tile, ic);
   const uint32_t tu_i = tile / (uint32_t)P.ntv;
   const int u0 = (int)tu_i * Tu, v0 = (int)(tile - tu_i * (uint32_t)P.ntv) * Tv;
   const float *gplane = grid + (size_t)ic * npol_g * P.n_u * P.n_v * 2;

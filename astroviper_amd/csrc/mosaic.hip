@@ -134,8 +134,9 @@ __global__ __launch_bounds__(64 * NPOL) void k_mosaic_grid(PlanDev P, MosaicArgs
   if (u >= n_units) return;
   const uint4 unit = P.gunits[u];
   const uint32_t b = unit.x, first = unit.y, cnt = unit.z, fl = unit.w;
-  const uint32_t tile_i = b / (uint32_t)P.n_img_chan;
-  const int ic = (int)(b - tile_i * (uint32_t)P.n_img_chan);
+  uint32_t tile_i;
+  int ic;
+  bin_parts(P, (uint32_t)b, tile_i, ic);
   const uint32_t tu_i = tile_i / (uint32_t)P.ntv;
   const int u0 = (int)tu_i * T, v0 = (int)(tile_i - tu_i * (uint32_t)P.ntv) * TV;
   const uint32_t prim_end = P.bin_start[b] + P.cnt_prim[b];

@@ -8,7 +8,14 @@
 // overlaps ("duplicate" records), so that each tile of the grid is produced
 // by exactly one owner with no halo exchange.  Within a bin, primary records
 // come first.  Bins are ordered tile-major, channel-minor, so neighbouring
-// channels of the same rows are processed close together in time.
+// channels of the same rows are processed close together in time; where rows
+// carry their own channel, channels share no samples, and bins are ordered
+// channel-major instead: the units at work at one time then gather from few
+// channels' samples, and a block of rows counts and places its records in one
+// stretch of bins (96 planes of 512 x 512 with 20 million samples, supports 9,
+// 7 and 5: FP32 gridders 715, 628 and 608 us channel-minor, 449, 419 and 416
+// channel-major; binning 432, 407 and 426 -> 347, 326 and 341, and 314, 300
+// and 304 with the block's own channel constants at hand).
 //
 // Binning is a counting sort.  The counts come from chunks (one channel, a
 // range of rows) gathered in LDS when a channel's tiles fit there, else from
@@ -99,7 +106,7 @@ __device__ inline void sample_geometry(const PlanDev &P, int64_t row, int chan, 
 }
 
 __device__ inline int64_t bin_of(const PlanDev &P, int tu, int tv, int ic) {
-  return ((int64_t)tu * P.ntv + tv) * P.n_img_chan + ic;
+  return bin_number(P, (int64_t)tu * P.ntv + tv, ic);
 }
 
 // One channel's constants into the plan.
@@ -359,22 +366,73 @@ __global__ __launch_bounds__(kChunkThreads) void k_count_chunks(PlanDev P, const
 // row-chunk, channel by channel within one: the channels of a row, which
 // share cache lines, then lie a run apart in the bin instead of a whole
 // channel's records apart.
+// With `ident` every channel is its own image channel.
+// f(i, n) takes n <= kRunBatch runs, the first at i and the others ntiles
+// apart: their loads go out together.
+constexpr int kRunBatch = 8;
 template <typename F>
-__device__ inline void chunk_runs(const PlanDev &P, int ic, int t, int seg, int nseg, F f) {
+__device__ inline void chunk_runs(const PlanDev &P, bool ident, int ic, int t, int seg, int nseg,
+                                  F f) {
   const int ntiles = P.ntu * P.ntv, K = P.chunks_per_chan;
   const int k0 = (int)((int64_t)K * seg / nseg), k1 = (int)((int64_t)K * (seg + 1) / nseg);
   if (P.chunk_all) {
-    for (int k = k0; k < k1; ++k) f((int64_t)k * ntiles + t);
+    for (int k = k0; k < k1; k += kRunBatch)
+      f((int64_t)k * ntiles + t, min(kRunBatch, k1 - k));
   } else if (P.n_img_chan < P.n_chan) {
     for (int k = k0; k < k1; ++k)
       for (int c = 0; c < P.n_chan; ++c)
-        if (P.chan_map[c] == ic) f(((int64_t)c * K + k) * ntiles + t);
+        if (P.chan_map[c] == ic) f(((int64_t)c * K + k) * ntiles + t, 1);
   } else {
-    for (int c = 0; c < P.n_chan; ++c) {
-      if (P.chan_map[c] != ic) continue;
-      for (int k = k0; k < k1; ++k) f(((int64_t)c * K + k) * ntiles + t);
+    for (int c = ident ? ic : 0; c < (ident ? ic + 1 : P.n_chan); ++c) {
+      if (!ident && P.chan_map[c] != ic) continue;
+      for (int k = k0; k < k1; k += kRunBatch)
+        f(((int64_t)c * K + k) * ntiles + t, min(kRunBatch, k1 - k));
     }
   }
+}
+
+// Whether every channel is its own image channel, found by a whole wavefront.
+__device__ inline bool chan_identity(const PlanDev &P) {
+  bool same = P.n_img_chan == P.n_chan;
+  for (int c = (int)__lane_id(); same && c < P.n_chan; c += 64) same = P.chan_map[c] == c;
+  return __all(same);
+}
+
+// Counts of a batch of runs added to (sp, sd).
+__device__ inline void add_runs(const PlanDev &P, int64_t i, int n, uint32_t &sp, uint32_t &sd) {
+  const int ntiles = P.ntu * P.ntv;
+  uint32_t np[kRunBatch], nd[kRunBatch];
+#pragma unroll
+  for (int u = 0; u < kRunBatch; ++u) {  // unconditional loads: all in flight
+    np[u] = P.chunk_hist[i + (int64_t)min(u, n - 1) * ntiles];
+    nd[u] = P.chunk_dup[i + (int64_t)min(u, n - 1) * ntiles];
+  }
+#pragma unroll
+  for (int u = 0; u < kRunBatch; ++u) {
+    sp += u < n ? np[u] : 0u;
+    sd += u < n ? nd[u] : 0u;
+  }
+}
+
+// The first slots of a batch of runs written over their counts; (sp, sd) are
+// the first free slots before and after.
+__device__ inline void place_runs(const PlanDev &P, int64_t i, int n, uint32_t &sp,
+                                  uint32_t &sd) {
+  const int ntiles = P.ntu * P.ntv;
+  uint32_t np[kRunBatch], nd[kRunBatch];
+#pragma unroll
+  for (int u = 0; u < kRunBatch; ++u) {
+    np[u] = P.chunk_hist[i + (int64_t)min(u, n - 1) * ntiles];
+    nd[u] = P.chunk_dup[i + (int64_t)min(u, n - 1) * ntiles];
+  }
+#pragma unroll
+  for (int u = 0; u < kRunBatch; ++u)
+    if (u < n) {
+      P.chunk_hist[i + (int64_t)u * ntiles] = sp;
+      P.chunk_dup[i + (int64_t)u * ntiles] = sd;
+      sp += np[u];
+      sd += nd[u];
+    }
 }
 
 // Chunked pass 2: the counts of every bin, summed over the chunks of the
@@ -388,12 +446,10 @@ __global__ void k_chunk_totals(PlanDev P) {
   const int nbt = (P.ntu * P.ntv + kSegTiles - 1) / kSegTiles;
   const int ic = blockIdx.x / nbt, t = (blockIdx.x - ic * nbt) * kSegTiles + threadIdx.x;
   const int seg = threadIdx.y, nseg = blockDim.y;
+  const bool ident = chan_identity(P);
   uint32_t sp = 0, sd = 0;
   if (t < P.ntu * P.ntv)
-    chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
-      sp += P.chunk_hist[i];
-      sd += P.chunk_dup[i];
-    });
+    chunk_runs(P, ident, ic, t, seg, nseg, [&](int64_t i, int n) { add_runs(P, i, n, sp, sd); });
   part[0][seg][threadIdx.x] = sp;
   part[1][seg][threadIdx.x] = sd;
   __syncthreads();
@@ -402,7 +458,7 @@ __global__ void k_chunk_totals(PlanDev P) {
     sp += part[0][k][threadIdx.x];
     sd += part[1][k][threadIdx.x];
   }
-  const int64_t b = (int64_t)t * P.n_img_chan + ic;
+  const int64_t b = bin_number(P, t, ic);
   P.cnt_prim[b] = sp;
   P.cnt_all[b] = sp + sd;
 }
@@ -415,31 +471,23 @@ __global__ void k_chunk_bases(PlanDev P) {
   const int nbt = (P.ntu * P.ntv + kSegTiles - 1) / kSegTiles;
   const int ic = blockIdx.x / nbt, t = (blockIdx.x - ic * nbt) * kSegTiles + threadIdx.x;
   const int seg = threadIdx.y, nseg = blockDim.y;
+  const bool ident = chan_identity(P);
   const bool on = t < P.ntu * P.ntv;
   uint32_t sp = 0, sd = 0;
   if (on && nseg > 1)
-    chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
-      sp += P.chunk_hist[i];
-      sd += P.chunk_dup[i];
-    });
+    chunk_runs(P, ident, ic, t, seg, nseg, [&](int64_t i, int n) { add_runs(P, i, n, sp, sd); });
   part[0][seg][threadIdx.x] = sp;
   part[1][seg][threadIdx.x] = sd;
   __syncthreads();
   if (!on) return;
-  const int64_t b = (int64_t)t * P.n_img_chan + ic;
+  const int64_t b = bin_number(P, t, ic);
   sp = P.bin_start[b];
   sd = sp + P.cnt_prim[b];
   for (int k = 0; k < seg; ++k) {
     sp += part[0][k][threadIdx.x];
     sd += part[1][k][threadIdx.x];
   }
-  chunk_runs(P, ic, t, seg, nseg, [&](int64_t i) {
-    const uint32_t np = P.chunk_hist[i], nd = P.chunk_dup[i];
-    P.chunk_hist[i] = sp;
-    P.chunk_dup[i] = sd;
-    sp += np;
-    sd += nd;
-  });
+  chunk_runs(P, ident, ic, t, seg, nseg, [&](int64_t i, int n) { place_runs(P, i, n, sp, sd); });
 }
 
 // Slots for one record per lane from the LDS cursors `cur` (key: the tile,
@@ -553,7 +601,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_chunks(PlanDev P) {
 }
 
 // ---- row-block binning (rows carry their own channel) ---------------------
-// A workgroup takes kRowBlockRows consecutive rows.  Rows of one plane are
+// A workgroup takes row_block_rows consecutive rows.  Rows of one plane are
 // normally stored together, so the records of the block's "own" image
 // channel (that of its first row) are gathered per tile in LDS and reach the
 // global bins with one atomic per tile the block touches; the records of any
@@ -569,20 +617,33 @@ __device__ inline int row_image_channel(const PlanDev &P, int64_t row) {
   return (ic >= 0 && ic < P.n_img_chan) ? ic : -1;
 }
 
+// Geometry of a row that carries its channel, most often the block's own,
+// whose constants are at hand.
+__device__ inline void row_geometry(const PlanDev &P, int64_t row, const ChanGeo &own,
+                                    ItemGeo &g) {
+  const int c = P.row_chan[row];
+  const double uu = P.uvw[row * 3 + 0], vv = P.uvw[row * 3 + 1];
+  if (c == own.chan)
+    sample_geometry_at(P, row, own, uu, vv, g);
+  else
+    sample_geometry_at(P, row, chan_geo(P, c), uu, vv, g);
+}
+
 // Row-block pass 1: per-tile counts, (primaries) | (duplicates << 16); a row
 // adds at most two primaries and one duplicate to a tile and a block has
-// kRowBlockRows < 32768 rows, so neither half overflows.
+// at most kMaxRowBlockRows < 32768 rows, so neither half overflows.
 __global__ __launch_bounds__(kChunkThreads) void k_count_rows(PlanDev P) {
   extern __shared__ uint32_t h[];  // [n_tiles]
-  const int64_t r0 = (int64_t)blockIdx.x * kRowBlockRows;
+  const int64_t r0 = (int64_t)blockIdx.x * P.row_block_rows;
   const int ntiles = P.ntu * P.ntv;
   const int own = row_image_channel(P, r0);
+  const ChanGeo own_geo = chan_geo(P, r0 < P.n_rows ? P.row_chan[r0] : -1);
   for (int i = threadIdx.x; i < ntiles; i += blockDim.x) h[i] = 0u;
   __syncthreads();
-  for (int64_t row = r0 + threadIdx.x; row < r0 + kRowBlockRows; row += blockDim.x) {
+  for (int64_t row = r0 + threadIdx.x; row < r0 + P.row_block_rows; row += blockDim.x) {
     ItemGeo g;
     g.gvalid = g.dvalid = false;
-    if (row < P.n_rows) sample_geometry(P, row, 0, g);
+    if (row < P.n_rows) row_geometry(P, row, own_geo, g);
     write_masks(P, row, 0, g.gvalid, g.dvalid);
     if (!(g.gvalid || g.dvalid)) continue;
     const RecPlan rp = record_plan(P, g);
@@ -605,7 +666,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_count_rows(PlanDev P) {
     const uint32_t hv = h[i];
     keep[i] = hv;
     if (!hv) continue;
-    const int64_t b = (int64_t)i * P.n_img_chan + own;
+    const int64_t b = bin_number(P, i, own);
     const uint32_t np = hv & 0xFFFFu;
     if (np) atomicAdd(&P.cnt_prim[b], np);
     atomicAdd(&P.cnt_all[b], np + (hv >> 16));
@@ -620,9 +681,10 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_rows(PlanDev P) {
   extern __shared__ uint32_t lds[];
   const int ntiles = P.ntu * P.ntv;
   uint32_t *cp = lds, *cd = lds + ntiles;  // [n_tiles] each
-  const int64_t r0 = (int64_t)blockIdx.x * kRowBlockRows;
-  const int64_t r1 = min(r0 + (int64_t)kRowBlockRows, P.n_rows);
+  const int64_t r0 = (int64_t)blockIdx.x * P.row_block_rows;
+  const int64_t r1 = min(r0 + (int64_t)P.row_block_rows, P.n_rows);
   const int own = row_image_channel(P, r0);
+  const ChanGeo own_geo = chan_geo(P, r0 < P.n_rows ? P.row_chan[r0] : -1);
   if (own >= 0) {
     const uint32_t *kept = P.row_hist + (int64_t)blockIdx.x * ntiles;
     for (int i = threadIdx.x; i < ntiles; i += blockDim.x) {
@@ -632,7 +694,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_rows(PlanDev P) {
     }
     __syncthreads();
     for (int i = threadIdx.x; i < ntiles; i += blockDim.x) {
-      const int64_t b = (int64_t)i * P.n_img_chan + own;
+      const int64_t b = bin_number(P, i, own);
       if (cp[i]) cp[i] = atomicAdd(&P.cur_prim[b], cp[i]);
       if (cd[i]) cd[i] = atomicAdd(&P.cur_dup[b], cd[i]);
     }
@@ -640,7 +702,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_rows(PlanDev P) {
   }
   for (int64_t row = r0 + threadIdx.x; row < r1; row += blockDim.x) {
     ItemGeo g;
-    sample_geometry(P, row, 0, g);
+    row_geometry(P, row, own_geo, g);
     if (!(g.gvalid || g.dvalid)) continue;
     const RecPlan rp = record_plan(P, g);
     if (g.ic != own) {
@@ -666,15 +728,17 @@ __global__ __launch_bounds__(kChunkThreads) void k_scatter_rows(PlanDev P) {
 
 // Pair units: the bins of tiles 2j and 2j + 1 (along v) of pair p, and the
 // primary records of both.
-__device__ inline void pair_bins(const PlanDev &P, int64_t p, int64_t &b0, bool &has1,
-                                 uint32_t &n) {
+__device__ inline void pair_bins(const PlanDev &P, int64_t p, int64_t &b0, int64_t &b1,
+                                 bool &has1, uint32_t &n) {
   const int ntv2 = (P.ntv + 1) / 2;
-  const int64_t tp = p / P.n_img_chan;
-  const int ic = (int)(p - tp * P.n_img_chan);
+  const int64_t per = P.chan_major ? (int64_t)P.ntu * ntv2 : P.n_img_chan, q = p / per;
+  const int64_t tp = P.chan_major ? p - q * per : q;
+  const int ic = (int)(P.chan_major ? q : p - q * per);
   const int tu = (int)(tp / ntv2), tv = 2 * (int)(tp - (int64_t)tu * ntv2);
-  b0 = ((int64_t)tu * P.ntv + tv) * P.n_img_chan + ic;
+  b0 = bin_of(P, tu, tv, ic);
   has1 = tv + 1 < P.ntv;
-  n = P.cnt_prim[b0] + (has1 ? P.cnt_prim[b0 + P.n_img_chan] : 0u);
+  b1 = has1 ? bin_of(P, tu, tv + 1, ic) : b0;
+  n = P.cnt_prim[b0] + (has1 ? P.cnt_prim[b1] : 0u);
 }
 
 // ---- bin offsets and work units --------------------------------------------
@@ -723,10 +787,10 @@ __device__ inline void bin_values(const PlanDev &P, int64_t b, uint32_t (&v)[3])
 }
 
 __device__ inline uint32_t pair_value(const PlanDev &P, int64_t p) {
-  int64_t b0;
+  int64_t b0, b1;
   bool has1;
   uint32_t n;
-  pair_bins(P, p, b0, has1, n);
+  pair_bins(P, p, b0, b1, has1, n);
   const uint32_t cap = (uint32_t)P.unit_cap;
   return (n + cap - 1) / cap;
 }
@@ -773,10 +837,10 @@ __device__ inline void index_pairs(const PlanDev &P, int64_t p0, int64_t p1, uin
   for (int64_t base = p0; base < p1; base += blockDim.x) {
     const int64_t p = base + threadIdx.x;
     const bool on = p < p1;
-    int64_t b0 = 0;
+    int64_t b0 = 0, b1 = 0;
     bool has1 = false;
     uint32_t n = 0u;
-    if (on) pair_bins(P, p, b0, has1, n);
+    if (on) pair_bins(P, p, b0, b1, has1, n);
     const uint32_t nu = (n + cap - 1) / cap;
     uint32_t v[1] = {nu}, total[1];
     block_scan_n<1>(v, total, sh);
@@ -784,9 +848,9 @@ __device__ inline void index_pairs(const PlanDev &P, int64_t p0, int64_t p1, uin
     carry += total[0];
     if (!on) continue;
     P.punit_start[p] = k0;
-    const uint32_t b1 = has1 ? (uint32_t)(b0 + P.n_img_chan) : kNoBin;
+    const uint32_t second = has1 ? (uint32_t)b1 : kNoBin;
     for (uint32_t k = 0; k < nu; ++k)
-      P.punits[k0 + k] = make_uint4((uint32_t)b0, k * cap, min(cap, n - k * cap), b1);
+      P.punits[k0 + k] = make_uint4((uint32_t)b0, k * cap, min(cap, n - k * cap), second);
   }
 }
 
@@ -803,14 +867,14 @@ __device__ inline void index_ends(const PlanDev &P, const uint32_t (&carry)[3]) 
 // samples, binned in 21 launches: 85 us; in three: 32 us).
 __global__ __launch_bounds__(1024) void k_index_small(PlanDev P) {
   __shared__ uint32_t sh[16 * 3];
+  const bool ident = chan_identity(P);
   if (P.chunked && !P.row_chan) {
     for (int64_t b = threadIdx.x; b < P.n_bins; b += blockDim.x) {
-      const int t = (int)(b / P.n_img_chan), ic = (int)(b - (int64_t)t * P.n_img_chan);
+      uint32_t t;
+      int ic;
+      bin_parts(P, (uint32_t)b, t, ic);
       uint32_t sp = 0, sd = 0;
-      chunk_runs(P, ic, t, 0, 1, [&](int64_t i) {
-        sp += P.chunk_hist[i];
-        sd += P.chunk_dup[i];
-      });
+      chunk_runs(P, ident, ic, (int)t, 0, 1, [&](int64_t i, int n) { add_runs(P, i, n, sp, sd); });
       P.cnt_prim[b] = sp;
       P.cnt_all[b] = sp + sd;
     }
@@ -826,15 +890,11 @@ __global__ __launch_bounds__(1024) void k_index_small(PlanDev P) {
   if (P.chunk_scatter) {
     __syncthreads();
     for (int64_t b = threadIdx.x; b < P.n_bins; b += blockDim.x) {
-      const int t = (int)(b / P.n_img_chan), ic = (int)(b - (int64_t)t * P.n_img_chan);
+      uint32_t t;
+      int ic;
+      bin_parts(P, (uint32_t)b, t, ic);
       uint32_t sp = P.bin_start[b], sd = sp + P.cnt_prim[b];
-      chunk_runs(P, ic, t, 0, 1, [&](int64_t i) {
-        const uint32_t np = P.chunk_hist[i], nd = P.chunk_dup[i];
-        P.chunk_hist[i] = sp;
-        P.chunk_dup[i] = sd;
-        sp += np;
-        sd += nd;
-      });
+      chunk_runs(P, ident, ic, (int)t, 0, 1, [&](int64_t i, int n) { place_runs(P, i, n, sp, sd); });
     }
   }
 }
@@ -842,7 +902,7 @@ __global__ __launch_bounds__(1024) void k_index_small(PlanDev P) {
 // General path: per-block sums (kIndexSpan bins or pairs a block), one
 // workgroup that scans them in place, then the offsets and units block by
 // block.  scan_tmp: [3][bin blocks] then [pair blocks].
-constexpr int kIndexSpan = 4096;
+constexpr int kIndexSpan = 1024;
 __global__ __launch_bounds__(1024) void k_index_sums(PlanDev P, int nb_blocks) {
   __shared__ uint32_t sh[16 * 3];
   const bool pairs = (int)blockIdx.x >= nb_blocks;
@@ -903,8 +963,11 @@ __global__ __launch_bounds__(1024) void k_index_apply(PlanDev P, int nb_blocks) 
   index_bins(P, blk * kIndexSpan, min((blk + 1) * (int64_t)kIndexSpan, P.n_bins), carry, sh);
 }
 
-// Segments of the chunk totals and bases passes: about eight runs each.
+// Segments of the chunk totals and bases passes: about eight runs each, one
+// where the bins alone fill the chip (a second pass over the counts of a
+// million bins: 62 -> 227 us).
 static int chunk_segments(const PlanDev &d) {
+  if (d.n_bins >= 1 << 16) return 1;
   const int64_t runs =
       (int64_t)d.chunks_per_chan * (d.chunk_all ? 1 : d.n_chan) / d.n_img_chan;
   return (int)std::max<int64_t>(
@@ -1077,6 +1140,8 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.ntu = (n_u + tile_u - 1) / tile_u;
   d.ntv = (n_v + tile_v - 1) / tile_v;
   d.n_bins = (int64_t)d.ntu * d.ntv * n_img_chan;
+  d.chan_major = row_channels && d.n_bins < ((int64_t)1 << 32);
+  d.bin_minor = d.chan_major ? (uint32_t)(d.ntu * d.ntv) : (uint32_t)n_img_chan;
   d.n_items = n_items;
   // a footprint overlaps at most 2x2 tiles, plus one separate degrid record
   d.max_records = 5 * n_items;
@@ -1102,9 +1167,16 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   const int64_t chunk_cells =
       d.chunked ? (int64_t)(d.chunk_all ? 1 : n_chan) * d.chunks_per_chan * ntiles : 0;
   // row-block counts, kept for plans whose rows carry their channel when a
-  // block's counters and cursors fit in 160 KB of LDS
+  // block's counters and cursors fit in 160 KB of LDS.  Blocks as the chunks:
+  // about kChunkTarget of them, at least half a row per tile, and few enough
+  // rows for 16-bit counts
+  d.row_block_rows = (int32_t)(
+      std::min<int64_t>(kMaxRowBlockRows / kChunkThreads,
+                        std::max<int64_t>(1, (std::max(n_rows / kChunkTarget, ntiles / 2) +
+                                              kChunkThreads - 1) / kChunkThreads)) *
+      kChunkThreads);
   const int64_t row_cells = (row_channels && n_rows > 0 && 8 * ntiles <= 160 * 1024)
-                                ? (n_rows + kRowBlockRows - 1) / kRowBlockRows * ntiles
+                                ? (n_rows + d.row_block_rows - 1) / d.row_block_rows * ntiles
                                 : 0;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -1234,14 +1306,14 @@ int av_plan_set_uvw(av_plan *plan, const double *uvw, const double *freq,
     else d.chunk_scatter = fits;
   }
   const int64_t nchunks = (int64_t)(d.chunk_all ? 1 : d.n_chan) * d.chunks_per_chan;
-  const unsigned row_grid = (unsigned)((d.n_rows + kRowBlockRows - 1) / kRowBlockRows);
+  const unsigned row_grid = (unsigned)((d.n_rows + d.row_block_rows - 1) / d.row_block_rows);
   const bool by_chunks = d.chunked && !row_chan;
   if (!by_chunks) {  // the counting pass of chunks sets its channels up itself
     hipLaunchKernelGGL(k_chan_setup, dim3((d.n_chan + 255) / 256), dim3(256), 0, s, d, freq,
                        chan_map);
     AV_LAUNCH_CHECK("k_chan_setup");
-    if ((rc = launch_fill_u32(d.cnt_all, 0u, d.n_bins, s))) return rc;
-    if ((rc = launch_fill_u32(d.cnt_prim, 0u, d.n_bins, s))) return rc;
+    // both counts in one fill: they lie one after the other in the plan
+    if ((rc = launch_fill_u32(d.cnt_all, 0u, d.cnt_prim - d.cnt_all + d.n_bins, s))) return rc;
   }
   // pass 1: counts per bin, or per chunk and tile
   if (d.row_blocks) {

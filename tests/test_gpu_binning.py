@@ -108,3 +108,71 @@ def test_compensated_sums_of_split_bins(gpu, oracle, cap, tile):
     assert _rel(g2.cpu().numpy(), 2 * gref) < 16 * 2.0 ** -24
     assert _rel(sw2.cpu().numpy(), 2 * swref) < 1e-12
     plan.close()
+
+
+@pytest.mark.parametrize("chan_map,n_img", [
+    ([2, 0, 1, 4, 3], 5),          # a permutation
+    ([1, 1, 0, 0, 2, 1, 2], 3),    # channels averaged into three
+    ([0, -1, 0, 5, 0], 1),         # some mapped outside the grid
+    ([3, 0, 0, 6, 1, 2, 5, 4], 8),  # as many image channels, not one to one
+])
+@pytest.mark.parametrize("n_u", [96, 1040])
+def test_channel_maps(gpu, oracle, chan_map, n_img, n_u):
+    from astroviper_amd.device import GridPlan
+    nt, nb, nchan, n_uv = 6, 67, len(chan_map), (n_u, n_u)
+    uvw, freq, vis, w, flag, cell = _samples(nt, nb, nchan, 1, n_uv, 17)
+    cube, sw = oracle.standard_grid(vis, uvw, np.where(flag, 0, w), freq, n_uv, cell,
+                                    chan_mode="cube")
+    gref = np.zeros((n_img,) + cube.shape[1:], dtype=complex)
+    swref = np.zeros((n_img, 1))
+    for c, ic in enumerate(chan_map):
+        if 0 <= ic < n_img:
+            gref[ic] += cube[c]
+            swref[ic] += sw[c]
+    rows = nt * nb
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(rows, nchan, n_img, n_uv, cell, device=gpu, n_baseline=nb)
+    plan.set_uvw(dev(uvw.reshape(rows, 3)), dev(freq), dev(np.array(chan_map, dtype=np.int32)))
+    g, s = plan.grid(dev(vis.reshape(-1, 1)), dev(w.reshape(-1, 1)),
+                     dev(flag.reshape(-1, 1).astype(np.uint8)))
+    assert _rel(g.cpu().numpy(), gref) < 1e-12
+    assert _rel(s.cpu().numpy(), swref) < 1e-12
+    plan.close()
+
+
+@pytest.mark.parametrize("n_rows,order", [(1, "sorted"), (63, "mixed"), (5000, "sorted"),
+                                          (5000, "mixed"), (1 << 21, "sorted")])
+def test_rows_with_their_own_channel(gpu, oracle, n_rows, order):
+    """Blocks of rows of one channel, of several, and of out-of-range ones."""
+    from astroviper_amd.device import GridPlan
+    rng = np.random.default_rng(n_rows)
+    n_uv, nchan, cell = (96, 112), 5, (-1e-4, 1e-4)
+    freq = np.linspace(1.0e9, 1.3e9, nchan)
+    uvw = rng.uniform(-1100.0, 1100.0, size=(n_rows, 3))
+    chan = rng.integers(-1, nchan + 1, size=n_rows)
+    if order == "sorted":
+        chan = np.sort(chan)
+    vis = rng.standard_normal(n_rows) + 1j * rng.standard_normal(n_rows)
+    w = rng.uniform(0.5, 1.5, size=n_rows)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(n_rows, nchan, nchan, n_uv, cell, device=gpu, row_channels=True)
+    plan.set_uvw(dev(uvw), dev(freq), None, dev(chan.astype(np.int32)))
+    g, s = plan.grid(dev(vis.reshape(-1, 1)), dev(w.reshape(-1, 1)))
+    m = plan.degrid(g).cpu().numpy()[:, 0]
+    g, s = g.cpu().numpy(), s.cpu().numpy()
+    plan.close()
+    for c in range(nchan):
+        r = chan == c
+        if not r.any():
+            assert not g[c].any()
+            continue
+        shape = (1, int(r.sum()), 1, 1)
+        gref, sref = oracle.standard_grid(vis[r].reshape(shape), uvw[r].reshape(1, -1, 3),
+                                          w[r].reshape(shape), freq[c:c + 1], n_uv, cell,
+                                          chan_mode="cube")
+        if np.abs(gref).max() > 0:
+            assert _rel(g[c], gref[0]) < 1e-12 and _rel(s[c], sref[0]) < 1e-12
+            mref = oracle.degrid(uvw[r].reshape(1, -1, 3), np.zeros(shape, bool), freq[c:c + 1],
+                                 gref, cell)
+            assert _rel(m[r], mref.ravel()) < 1e-12
+    assert not m[(chan < 0) | (chan >= nchan)].any()
