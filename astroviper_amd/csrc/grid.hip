@@ -551,8 +551,22 @@ constexpr int grid_mfma_min_blocks() {
   return (sizeof(R) == 4 && !COMP && MB * 2 * NPOL * VB <= 8) ? 6 : 1;
 }
 
+// Wavefronts of a workgroup, at most.  An FP64 weight table takes 33 KB of LDS
+// at support 7 and oversampling 100, so workgroups of four leave three
+// wavefronts to a SIMD; eight share a table where there are units enough for
+// every compute unit (twice over): 643 -> 585 us for 4.8 M samples x 2
+// polarisations on 16 planes of 1024^2, but 36 -> 42 us for a snapshot's 256
+// tiles, whose workgroups of eight leave most of the chip idle.
+constexpr int kGridWideWaves = 8;
+constexpr int64_t kGridWideUnits = 4096;
+template <typename R>
+constexpr int grid_mfma_max_waves() {
+  return sizeof(R) == 8 ? kGridWideWaves : kGridMaxWaves;
+}
+
 template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF>
-__global__ __launch_bounds__(kGridThreads, (grid_mfma_min_blocks<R, NPOL, MB, VB, COMP>()))
+__global__ __launch_bounds__(64 * grid_mfma_max_waves<R>(),
+                             (grid_mfma_min_blocks<R, NPOL, MB, VB, COMP>()))
 void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
                                                             const R *__restrict__ weight,
                                                             const uint8_t *__restrict__ flag,
@@ -582,15 +596,15 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
   // 16 workgroups of 4 units: the 64 channels of a tile under one L2
   // (compensated: a workgroup per unit, that of a group's first unit sums the
   // whole group)
-  constexpr int kUnitsPerWg = COMP ? 1 : kGridMaxWaves;
-  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup * kGridMaxWaves / kUnitsPerWg);
-  if (blk * kUnitsPerWg >= n_units) return;  // whole workgroup idle
+  const uint32_t units_per_wg = COMP ? 1 : blockDim.x / 64;
+  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup * kGridMaxWaves / units_per_wg);
+  if (blk * units_per_wg >= n_units) return;  // whole workgroup idle
   copy_wtab_padded(tab, L, P);
   for (int i = tid; i < L.nnrm; i += blockDim.x) nrm[i] = P.nrm[i];
   __syncthreads();  // the only workgroup barrier: tables ready
   // the same for every lane: scalar registers for the unit and its bounds
   uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane(
-      (int)(COMP ? blk : blk * kGridMaxWaves + wave));
+      (int)(COMP ? blk : blk * units_per_wg + wave));
   if (u >= n_units) return;
 
   const int Tu = 16 * MB, Tv = 16 * VB;
@@ -745,11 +759,17 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
     fetch_raw<R, NPOL>(raw1, r1.x, vis, weight, flag, psf, adjoint);
     const uint2 r2 = load_record(P, base + 128 + lane, end);
     wave_lds_sync();
-    // ---- four records per matrix-core step
+    // ---- four records per matrix-core step, four steps at a time: each
+    // waits for two LDS reads in turn (the record's table bases, then its
+    // weights), which one step after another left unhidden at three
+    // wavefronts per SIMD (FP64: 755 us, four at a time 643, two 684, eight
+    // 653; see kGridWideWaves).  Steps past the last record add staged zeros.
     const int nst = (int)min((uint32_t)64, end - base);
     const int li_nw = li * L.nw;
-    for (int s4 = 0; s4 < nst; s4 += 4) {
-      const int rec = s4 + lk;
+    for (int s16 = 0; s16 < nst; s16 += 16)
+#pragma unroll
+    for (int s4 = 0; s4 < 16; s4 += 4) {
+      const int rec = s16 + s4 + lk;
       const uint32_t tb = st_geo[rec];
       const uint32_t tbu = tb & 0xFFFFu, tbv = tb >> 16;
       R a[MB], wv[VB];
@@ -1020,7 +1040,13 @@ static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
   const DeviceProps &prop = device_props();
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   const MfmaLds L = mfma_lds_layout<R, NPOL>(d.ov, d.support, 16 * (MB > VB ? MB : VB));
-  const int lds = L.total + mfma_comb_bytes<NPOL, MB, VB, COMP>();
+  int nw = kGridMaxWaves;
+  if constexpr (grid_mfma_max_waves<R>() > kGridMaxWaves) {
+    if (d.max_gunits >= kGridWideUnits &&
+        (size_t)(L.st_d + kGridWideWaves * L.wave_bytes) <= prop.lds_per_block)
+      nw = kGridWideWaves;
+  }
+  const int lds = L.st_d + nw * L.wave_bytes + mfma_comb_bytes<NPOL, MB, VB, COMP>();
   {
     const int rc_lds = ensure_lds_limit<k_grid_mfma<R, NPOL, MB, VB, COMP, PSF>>(lds, "av_grid: hipFuncSetAttribute");
     if (rc_lds) return rc_lds;
@@ -1032,11 +1058,11 @@ static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
                        (float *)grid, 0);
     AV_LAUNCH_CHECK("k_comp_slots");
   }
-  constexpr int kUnitsPerWg = COMP ? 1 : kGridMaxWaves;
+  const int units_per_wg = COMP ? 1 : nw;
   const unsigned nwg =
-      (unsigned)xcd_grouped_grid((d.max_gunits + kUnitsPerWg - 1) / kUnitsPerWg,
-                                 kGridXcdGroup * kGridMaxWaves / kUnitsPerWg);
-  hipLaunchKernelGGL(kfn, dim3(nwg), dim3(kGridThreads), lds, s, d, (const R *)vis,
+      (unsigned)xcd_grouped_grid((d.max_gunits + units_per_wg - 1) / units_per_wg,
+                                 kGridXcdGroup * kGridMaxWaves / units_per_wg);
+  hipLaunchKernelGGL(kfn, dim3(nwg), dim3(64 * nw), lds, s, d, (const R *)vis,
                      (const R *)weight, flag, cgk, (R *)grid, mode);
   AV_LAUNCH_CHECK("k_grid_mfma");
   if constexpr (COMP) {
