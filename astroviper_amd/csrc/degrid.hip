@@ -410,9 +410,14 @@ struct DegridGroup {
 // at most 8 column blocks (80 registers without spills; a 16 x 16 tile's
 // workgroup then needs 26,988 bytes of LDS, a sixth of the CU's 160 KB);
 // five for up to 12 blocks without halves (96 registers; at six the
-// one-polarisation kernels spill).  Other variants keep the compiler's choice.
+// one-polarisation kernels spill).  FP64: four with up to 4 blocks (128
+// registers; the compiler's choice of 156 left three: 4.8 M samples on 16
+// planes of 1024^2 take 465 us instead of 549 with two polarisations, 423
+// instead of 493 with one), three with up to 8 (742 instead of 947 with four
+// polarisations; at four 816).  Other variants keep the compiler's choice.
 template <typename R, int NB, int NBW>
 constexpr int degrid_mfma_min_blocks() {
+  if (sizeof(R) == 8) return NBW <= 4 ? 4 : NBW <= 8 ? 3 : 1;
   return (sizeof(R) == 4 && NBW < NB && NBW <= 8) ? 6 : (sizeof(R) == 4 && NB <= 12) ? 5 : 1;
 }
 
@@ -1435,6 +1440,14 @@ static int dispatch_degrid(av_plan *plan, const void *grid, int npol_g, const in
   }
   if (nb <= 4)
     return launch_degrid_mfma<R, NPOL, 4>(plan, grid, npol_g, pol_map, flag, cgk, vis_out, mode, s);
+  // two polarisations in FP64: records split by v, four of the six blocks
+  // (eight whole blocks, two of them padding, took 835 us where this takes
+  // 549, both at the compiler's choice of registers)
+  if constexpr (NPOL == 2 && sizeof(R) == 8)
+    if (nb <= 6 &&
+        degrid_halves_fit<R, NPOL, 6, 4>(plan->d.tile_u, plan->d.tile_v, plan->d.support))
+      return launch_degrid_mfma<R, NPOL, 6, 4>(plan, grid, npol_g, pol_map, flag, cgk, vis_out,
+                                               mode, s);
   if (nb <= 8)
     return launch_degrid_mfma<R, NPOL, 8>(plan, grid, npol_g, pol_map, flag, cgk, vis_out, mode, s);
   if (nb <= 12) {
