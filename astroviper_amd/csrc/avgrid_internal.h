@@ -44,7 +44,8 @@ constexpr int kMaxRowsPerChunk = 124 * kChunkThreads;  // rows of one chunked-bi
 constexpr int64_t kChunkTarget = 1024;  // chunks a plan is cut into when its rows allow
 constexpr int kChunkAllChans = 2;       // channels of a continuum plan whose chunks span them all
 constexpr int64_t kCapSamples = 12288;  // samples of a plan per record of its default unit cap
-constexpr int64_t kPackRows = 1 << 20;  // rows from which samples are packed (k_pack_samples)
+constexpr int64_t kPackSamples = 1 << 20;  // samples from which they are packed (k_pack_samples)
+constexpr int kPackLine = 32;  // polarisations x channels of a row that share lines without packing
 constexpr int kMaxRowBlockRows = 16 * kChunkThreads;  // rows of a row-block binning workgroup
 
 // Packed geometry of one sample relative to a tile origin:
@@ -226,9 +227,6 @@ struct PlanDev {
   // per grid unit, per polarisation: sum of weight * norm (FP64)
   double *upart;                    // [max_gunits * 4]
   uint32_t *counters;               // scratch for statistics
-  // kPackRows or more rows that carry their own channel, 16 x 16 tiles: room
-  // for the weighted samples of one polarisation, {re, im, weight, -}
-  float4 *pack;                     // [n_rows], or NULL
 };
 
 // The number of tile `tile`'s bin of image channel ic, and back.

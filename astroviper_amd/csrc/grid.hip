@@ -1135,33 +1135,58 @@ __host__ __device__ inline H3Lds h3_lds_layout(int ov, int support) {
   return L;
 }
 
-// The weighted samples of a plan whose rows carry their own channel, side by
-// side: k_grid_h3 then fetches one cache line per record instead of the
-// visibility's, the weight's and the flag's.  Such rows are samples of their
-// own, with no channels beside them to share a line with, and a bin gathers
-// them in no order.  Three lines a record kept the gridder at the memory's
-// rate: 6.9 M samples of random order took 377 us on 32 planes of 512^2, 688
-// on one of 2048^2; packed 266 and 334, this pass included (41 us, a copy's
-// rate).  Plans make room for it from kPackRows rows: fewer samples stay in
-// the L2s (1 M on 8 planes: 62.4 and 62.8 us; 0.3 M on 4: 33.5 and 36.5).
-// Rows already sorted by tile lose (6.9 M: 188 and 215 us), but observations
-// are written time by time, which visits the tiles in no order.
-__global__ __launch_bounds__(256) void k_pack_samples(const float *__restrict__ vis,
+// The weighted samples, data then weights side by side: k_grid_h3 then
+// fetches one cache line per record instead of the visibility's, the weight's
+// and the flag's.  With one or two polarisations a line holds sixteen or
+// eight visibilities, but a record uses one, and what could share it (the
+// channels of a row, a baseline's next times) seldom falls in one tile at one
+// time: three lines a record kept the gridder at the memory's rate.  7.3 M
+// samples of 1024^2 planes, this pass included: one channel 658 -> 326 us with
+// one polarisation, 735 -> 458 with two; 16 channels 456 -> 263 and 577 ->
+// 462; 64 channels x 0.8 M rows 3.11 -> 1.40 ms and 3.46 -> 2.58; 6.9 M rows in
+// random order on 32 planes of 512^2, 377 -> 266.
+// Fewer than kPackSamples samples stay in the L2s (1.2 M: 97 -> 82 us; 0.3 M
+// in random order: 33.5 -> 36.5).  Where one image channel gathers a row's
+// channels side by side and they fill a line of weights (kPackLine samples),
+// the lines are shared already (32 channels 319 us either way, 64 988 ->
+// 1149; 16 277 -> 218).  Four polarisations fill a line in fewer channels and
+// need more room than the plan has.
+// They lie after the plan's records, where the array has room for five a
+// sample; plans whose samples leave too little (more than four records each
+// with one polarisation, three with two) grid unpacked, as the kernel sees
+// for itself.
+__device__ inline float *packed_samples(const PlanDev &P) {
+  return (float *)(P.rec + 3 * (size_t)P.bin_start[P.n_bins]);
+}
+template <int NPOL>
+__device__ inline bool pack_fits(const PlanDev &P) {
+  return (int64_t)P.bin_start[P.n_bins] * 12 + P.n_items * (int64_t)(12 * NPOL) <=
+         P.max_records * 12;
+}
+
+template <int NPOL>
+__global__ __launch_bounds__(256) void k_pack_samples(PlanDev P, const float *__restrict__ vis,
                                                       const float *__restrict__ weight,
-                                                      const uint8_t *__restrict__ flag,
-                                                      int64_t n, float4 *__restrict__ out) {
+                                                      const uint8_t *__restrict__ flag) {
+  if (!pack_fits<NPOL>(P)) return;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const Cplx2<float> v = ((const Cplx2<float> *)vis)[i];
-    const float w = flag && flag[i] ? 0.f : weight[i];
-    out[i] = make_float4(v.re * w, v.im * w, w, 0.f);
-  }
+  float *out = packed_samples(P);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < P.n_items; i += stride)
+#pragma unroll
+    for (int p = 0; p < NPOL; ++p) {
+      const Cplx2<float> v = ((const Cplx2<float> *)vis)[i * NPOL + p];
+      const float w = flag && flag[i * NPOL + p] ? 0.f : weight[i * NPOL + p];
+      out[i * 3 * NPOL + 2 * p] = v.re * w;
+      out[i * 3 * NPOL + 2 * p + 1] = v.im * w;
+      out[i * 3 * NPOL + 2 * NPOL + p] = w;
+    }
 }
 
 template <int NPOL, bool PSF, bool PACKED>
-__global__ __launch_bounds__(kGridThreads, (NPOL == 4 ? 4 : 5))
-void k_grid_h3(PlanDev P, const float *__restrict__ vis, const float *__restrict__ weight,
-               const uint8_t *__restrict__ flag, float *__restrict__ grid, int mode) {
+__device__ __forceinline__ void grid_h3(const PlanDev &P, const float *__restrict__ vis,
+                                        const float *__restrict__ weight,
+                                        const uint8_t *__restrict__ flag,
+                                        float *__restrict__ grid, int mode) {
   constexpr int C = 2 * NPOL;
   extern __shared__ __align__(16) char smem[];
   const int S = P.support, sc = S / 2, ov = P.ov;
@@ -1253,11 +1278,15 @@ void k_grid_h3(PlanDev P, const float *__restrict__ vis, const float *__restrict
 #pragma unroll
   for (int p = 0; p < NPOL; ++p) sw[p] = 0.0;
 
+  const float *pack = PACKED ? packed_samples(P) : nullptr;
   const auto fetch = [&](RawSample<float, NPOL> &s, uint32_t item) {
     if constexpr (PACKED) {
-      const float4 t = P.pack[item];
-      s.vv[0] = Cplx<float>{t.x, t.y};
-      s.wv[0] = t.z;
+      const float *t = pack + (size_t)item * (3 * NPOL);
+#pragma unroll
+      for (int p = 0; p < NPOL; ++p) {
+        s.vv[p] = Cplx<float>{t[2 * p], t[2 * p + 1]};
+        s.wv[p] = t[2 * NPOL + p];
+      }
       s.fbits = 0;
     } else {
       fetch_raw<float, NPOL>(s, item, vis, weight, flag, PSF, adjoint);
@@ -1428,7 +1457,21 @@ void k_grid_h3(PlanDev P, const float *__restrict__ vis, const float *__restrict
   }
 }
 
-template <int NPOL, bool PSF, bool PACKED = false>
+// With PACK the samples are packed first, where they fit.
+template <int NPOL, bool PSF, bool PACK>
+__global__ __launch_bounds__(kGridThreads, (NPOL == 4 ? 4 : 5))
+void k_grid_h3(PlanDev P, const float *__restrict__ vis, const float *__restrict__ weight,
+               const uint8_t *__restrict__ flag, float *__restrict__ grid, int mode) {
+  if constexpr (PACK) {
+    if (pack_fits<NPOL>(P)) {
+      grid_h3<NPOL, PSF, true>(P, vis, weight, flag, grid, mode);
+      return;
+    }
+  }
+  grid_h3<NPOL, PSF, false>(P, vis, weight, flag, grid, mode);
+}
+
+template <int NPOL, bool PSF, bool PACK = false>
 static int launch_grid_h3(av_plan *plan, const void *vis, const void *weight,
                           const uint8_t *flag, void *grid, double *sumwt, int mode,
                           hipStream_t s) {
@@ -1436,18 +1479,18 @@ static int launch_grid_h3(av_plan *plan, const void *vis, const void *weight,
   const H3Lds L = h3_lds_layout<NPOL>(d.ov, d.support);
   {
     const int rc_lds =
-        ensure_lds_limit<k_grid_h3<NPOL, PSF, PACKED>>(L.total, "av_grid: hipFuncSetAttribute");
+        ensure_lds_limit<k_grid_h3<NPOL, PSF, PACK>>(L.total, "av_grid: hipFuncSetAttribute");
     if (rc_lds) return rc_lds;
   }
-  if constexpr (PACKED) {
-    const int64_t blocks = std::min<int64_t>((d.n_rows + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_pack_samples, dim3((unsigned)blocks), dim3(256), 0, s,
-                       (const float *)vis, (const float *)weight, flag, d.n_rows, d.pack);
+  if constexpr (PACK) {
+    const int64_t blocks = std::min<int64_t>((d.n_items + 255) / 256, 8192);
+    hipLaunchKernelGGL(k_pack_samples<NPOL>, dim3((unsigned)blocks), dim3(256), 0, s, d,
+                       (const float *)vis, (const float *)weight, flag);
     AV_LAUNCH_CHECK("k_pack_samples");
   }
   const unsigned nwg = (unsigned)xcd_grouped_grid(
       (d.max_gunits + kGridMaxWaves - 1) / kGridMaxWaves, kGridXcdGroup);
-  hipLaunchKernelGGL((k_grid_h3<NPOL, PSF, PACKED>), dim3(nwg), dim3(kGridThreads), L.total, s, d,
+  hipLaunchKernelGGL((k_grid_h3<NPOL, PSF, PACK>), dim3(nwg), dim3(kGridThreads), L.total, s, d,
                      (const float *)vis, (const float *)weight, flag, (float *)grid, mode);
   AV_LAUNCH_CHECK("k_grid_h3");
   if (!(mode & AV_GRID_ADJOINT)) {
@@ -1470,8 +1513,9 @@ static int try_grid_h3(av_plan *plan, const void *vis, const void *weight, const
   done = true;
   if (mode & AV_GRID_PSF)
     return launch_grid_h3<NPOL, true>(plan, vis, weight, flag, grid, sumwt, mode, s);
-  if constexpr (NPOL == 1) {
-    if (d.pack && d.row_chan && !(mode & AV_GRID_ADJOINT))
+  if constexpr (NPOL <= 2) {
+    if (d.n_items >= kPackSamples && !(mode & AV_GRID_ADJOINT) &&
+        !(d.chunk_all && d.n_chan * NPOL >= kPackLine))
       return launch_grid_h3<NPOL, false, true>(plan, vis, weight, flag, grid, sumwt, mode, s);
   }
   return launch_grid_h3<NPOL, false>(plan, vis, weight, flag, grid, sumwt, mode, s);

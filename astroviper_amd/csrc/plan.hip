@@ -1183,8 +1183,6 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   const int64_t row_cells = (row_channels && n_rows > 0 && 8 * ntiles <= 160 * 1024)
                                 ? (n_rows + d.row_block_rows - 1) / d.row_block_rows * ntiles
                                 : 0;
-  const bool pack =
-      row_channels && tile_u == 16 && tile_v == 16 && n_rows >= kPackRows && !compact;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     size_t o = off;
@@ -1205,8 +1203,7 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
          o_nrm = take(sizeof(double) * (2 * (oversampling / 2 + 2) + 1)),
          o_wt32 = take(sizeof(float) * (support + 2) * (2 * (oversampling / 2 + 2) + 1)),
          o_wt64 = take(sizeof(double) * (support + 2) * (2 * (oversampling / 2 + 2) + 1)),
-         o_upart = take(sizeof(double) * 4 * d.max_gunits), o_ctr = take(4 * 16),
-         o_pack = take(pack ? sizeof(float4) * n_rows : 0);
+         o_upart = take(sizeof(double) * 4 * d.max_gunits), o_ctr = take(4 * 16);
   *bytes = off;
   if (!base) return AV_OK;
   char *c = base;
@@ -1241,7 +1238,6 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   // the units' partial sums are written after them, by the gridder
   d.scan_tmp = (uint32_t *)d.upart;
   d.counters = (uint32_t *)(c + o_ctr);
-  d.pack = pack ? (float4 *)(c + o_pack) : nullptr;
   p->alloc_base = base;
   p->alloc_bytes = off;
   return AV_OK;
