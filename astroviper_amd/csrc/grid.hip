@@ -843,7 +843,7 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
 
   // ---- flush: lane holds rows MO::row(lane/16, r), column lane%16 of every block
   if constexpr (COMP) {
-    // a bin of several groups: into its FP64 slot, which k_comp_finish rounds
+    // a bin of several groups: into its FP64 slot, which k_comp_slots rounds
     // to the grid once
     double *slots = multi ? comp_slots(P, mfma_comb_bytes<NPOL, MB, VB, true>()) : nullptr;
     if (slots) {
