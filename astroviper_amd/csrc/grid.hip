@@ -27,6 +27,7 @@ constexpr int kGridThreads = 256;
 constexpr int kGridMaxWaves = kGridThreads / 64;
 constexpr int kCompChunkBatches = 4;  // compensated mode: fold every 4*64 records
 // compensated mode: records a workgroup sums, however short the plan's units
+// (rounded up to whole units)
 constexpr uint32_t kCompGroupRecords = 8192;
 constexpr int kGridXcdGroup = 16;     // matrix-core kernel: workgroups per XCD group
 constexpr int kGridSubtile = AV_GRID_SUBTILE;
@@ -116,13 +117,13 @@ __device__ inline uint2 load_record(const PlanDev &P, uint32_t idx, uint32_t end
 }
 
 // Compensated mode: the FP64 sums of split bins.  They lie in the unused end
-// of the plan's record array, one slot per kCompGroupRecords records: a bin
-// split into several groups holds more records than that, so
-// bin_start / kCompGroupRecords numbers its slot uniquely.  A sample has at
-// most four records (five with a degrid record of its own) of the five the
-// array has room for, and a slot at most 16 KB, two bytes per record, so the
-// slots fit whenever no sample has five; where they do not,
-// the groups add into the grid in FP32.
+// of the plan's record array, one slot per kCompGroupRecords records: a group
+// is no shorter than that (comp_group_units), so a bin split into several
+// groups holds more records, and bin_start / kCompGroupRecords numbers its slot
+// uniquely.  A sample has at most four records (five with a degrid record of
+// its own) of the five the array has room for, and a slot at most 16 KB, two
+// bytes per record, so the slots fit whenever no sample has five; where they do
+// not, the groups add into the grid in FP32.
 __device__ inline double *comp_slots(const PlanDev &P, int slot_bytes) {
   const uint64_t n_rec = P.bin_start[P.n_bins];
   const uint64_t used = (n_rec * 12 + 255) & ~(uint64_t)255;
@@ -130,13 +131,20 @@ __device__ inline double *comp_slots(const PlanDev &P, int slot_bytes) {
   return used + need <= (uint64_t)P.max_records * 12 ? (double *)((char *)P.rec + used) : nullptr;
 }
 
+// Units of a compensated group: the fewest that hold kCompGroupRecords records,
+// whatever the plan's cap (rounded down, a cap of 5000 would make groups of 5000
+// records, and two bins of 6500 side by side share a slot).
+__device__ inline uint32_t comp_group_units(uint32_t cap) {
+  return max(1u, (kCompGroupRecords + cap - 1) / cap);
+}
+
 // Compensated mode: the units of a bin are summed in groups of
-// kCompGroupRecords records.  True when unit {b, first} leads its group, of
+// comp_group_units.  True when unit {b, first} leads its group, of
 // n_in units and cnt records; `multi` when its bin has other groups.
 __device__ inline bool comp_group(const PlanDev &P, int64_t b, uint32_t first, uint32_t &n_in,
                                   uint32_t &cnt, bool &multi) {
   const uint32_t cap = (uint32_t)P.unit_cap;
-  const uint32_t per = max(1u, kCompGroupRecords / cap);
+  const uint32_t per = comp_group_units(cap);
   const uint32_t k = (first - P.bin_start[b]) / cap;
   const uint32_t n_units = P.gunit_start[b + 1] - P.gunit_start[b];
   n_in = min(per, n_units - k);
@@ -874,7 +882,7 @@ __global__ __launch_bounds__(256) void k_comp_slots(PlanDev P, float *grid, int 
   for (uint32_t w0 = (blockIdx.x * 4 + threadIdx.x / 64) * 64; w0 < n_units;
        w0 += gridDim.x * 256) {
     const uint4 mine = P.gunits[min(w0 + lane, n_units - 1)];
-    const uint32_t per = max(1u, kCompGroupRecords / (uint32_t)P.unit_cap);
+    const uint32_t per = comp_group_units((uint32_t)P.unit_cap);
     const bool lead = w0 + lane < n_units && (mine.w & kUnitMulti) && (mine.w & kUnitFirst) &&
                       P.gunit_start[mine.x + 1] - P.gunit_start[mine.x] > per;
     for (unsigned long long m = __ballot(lead); m; m &= m - 1) {

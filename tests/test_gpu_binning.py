@@ -176,3 +176,38 @@ def test_rows_with_their_own_channel(gpu, oracle, n_rows, order):
                                  gref, cell)
             assert _rel(m[r], mref.ravel()) < 1e-12
     assert not m[(chan < 0) | (chan >= nchan)].any()
+
+
+@pytest.mark.parametrize("cap,per_tile,npol", [
+    (3000, 6500, 1), (3000, 6500, 2), (5000, 6500, 1), (6000, 6500, 4), (100, 8150, 1),
+    (8191, 8192, 1), (4096, 8193, 1),
+])
+def test_compensated_sums_of_neighbouring_split_bins(gpu, oracle, cap, per_tile, npol):
+    """Unit caps that do not divide the records of a compensated group, on
+    neighbouring tiles of equally many records, each in one tile only: a tile
+    that took another's sums would be off by its own size.  The sums are of
+    terms of one sign, in two groups at most: the bound of the test above."""
+    from astroviper_amd.device import GridPlan
+    n, tiles = 64, 16
+    rng = np.random.default_rng(cap + npol)
+    # 4 pixels about every tile's centre: footprints of 7 stay inside
+    at = np.repeat(np.arange(tiles), per_tile)
+    px = np.stack([16 * (at // 4), 16 * (at % 4)], 1) + 8 + rng.uniform(-4, 4, (at.size, 2))
+    px = px[rng.permutation(at.size)]
+    freq, cell = np.array([1.2e9]), 1e-4
+    scale = -(freq[0] * np.array([-cell, cell]) * n) / C
+    uvw = np.concatenate([(px - n // 2) / scale, np.zeros((at.size, 1))], 1)
+    w = rng.uniform(0.5, 1.5, (at.size, npol)).astype(np.float32)
+    gref, swref = oracle.standard_grid(None, uvw[:, None], w[:, None, None].astype(float), freq,
+                                       (n, n), (-cell, cell), chan_mode="cube", do_psf=True)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(at.size, 1, 1, (n, n), (-cell, cell), unit_cap=cap, device=gpu)
+    plan.set_uvw(dev(uvw), dev(freq))
+    st = plan.stats()
+    assert st["records"] == tiles * per_tile and st["bins"] == tiles
+    g, sw = plan.grid(None, dev(w), psf=True, compensated=True)
+    assert _rel(g.cpu().numpy(), gref) < 8 * 2.0 ** -24
+    assert _rel(sw.cpu().numpy(), swref) < 1e-12
+    g, sw = plan.grid(None, dev(w), grid=g, sumwt=sw, psf=True, accumulate=True, compensated=True)
+    assert _rel(g.cpu().numpy(), 2 * gref) < 16 * 2.0 ** -24
+    plan.close()
