@@ -183,7 +183,9 @@ class ResidentImager:
         step = max(1, (1 << 28) // max(1, npol * self.ny * self.nx))
         for c0 in range(0, nch, step):
             c1 = min(nch, c0 + step)
-            r = dirty[c0:c1].reshape((-1,) + tuple(dirty.shape[2:])).to(clean_dtype, copy=True)
+            # a copy in plane order, also of images that are views of another
+            r = dirty[c0:c1].reshape((-1,) + tuple(dirty.shape[2:])).to(
+                clean_dtype, copy=True, memory_format=torch.contiguous_format)
             p = psf[c0:c1, 0].to(clean_dtype).contiguous()
             m = torch.zeros_like(r)
             iters[c0:c1] = H.clean_planes_device(r, p, m, npol, int(niter), gain, threshold,

@@ -141,3 +141,23 @@ def test_model_to_uv_matches_shifted_fft(gpu, shape, cdt):
     ref = np.fft.fftshift(np.fft.fft2(np.fft.ifftshift(z, axes=ax), axes=ax), axes=ax)
     got = model_to_uv(torch.from_numpy(z).to(gpu), getattr(torch, cdt)).cpu().numpy()
     assert rel(got, ref) < (1e-6 if cdt == "complex64" else 1e-13)
+
+
+def test_deconvolve_of_strided_images(gpu):
+    """Dirty images and PSFs that are views of other layouts: the components
+    of the contiguous copies, bit for bit."""
+    from astroviper_amd.major_cycle import ResidentImager
+    ms, n_uv, cell = dataset(seed=8, n_time=10)
+    im = ResidentImager(ms, n_uv, cell, chan_mode="cube")
+    dirty, psf = im.grid_visibilities("VISIBILITY"), im.make_psf()
+    for clean_dtype in (torch.float32, torch.float64):
+        views = [(dirty.transpose(-1, -2), psf.transpose(-1, -2)),
+                 (dirty.transpose(0, 1), psf),
+                 (dirty[..., ::2], psf[..., ::2])]
+        for d, p in views:
+            ref = im.deconvolve(d.contiguous(), p.contiguous(), 15, clean_dtype=clean_dtype)
+            got = im.deconvolve(d, p, 15, clean_dtype=clean_dtype)
+            assert int(got[2].min()) == 15
+            assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+            np.testing.assert_array_equal(got[2], ref[2])
+    im.close()
