@@ -392,6 +392,9 @@ __global__ __launch_bounds__(kFftThreads) void k_image_rows(FftShape S, int64_t 
       const double f = t.tu[u0 + c] * sw;
       v.x = v.x / (f * t.tv[2 * i]);
       v.y = v.y / (f * t.tv[2 * i + 1]);
+    } else if (sumwt) {
+      v.x = v.x / sw;
+      v.y = v.y / sw;
     }
     store_pair(dst + (int64_t)c * S.n_v + 2 * i, v.x, v.y);
   };

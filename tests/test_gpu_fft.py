@@ -105,3 +105,18 @@ def test_fft_sizes_left_to_torch(gpu):
     a = D.uv_to_image(g, None, torch.empty((16, 32), device=gpu), work)
     b = D.uv_to_image(g.clone(), None, torch.empty((16, 32), device=gpu), work)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("odt,tol", [(torch.float64, 1e-14), (torch.float32, 4 * 2.0 ** -24)])
+def test_sums_of_weights_without_taper(gpu, odt, tol):
+    """1 / sumwt and the taper are independent of each other."""
+    from astroviper_amd import device as D
+    n, m, planes = 30, 48, 3
+    rng = np.random.default_rng(4)
+    g = rng.standard_normal((planes, n, m)) + 1j * rng.standard_normal((planes, n, m))
+    sw = rng.uniform(2, 9, size=planes)
+    ref = np.fft.fftshift(np.fft.ifft2(np.fft.ifftshift(g, axes=AX), axes=AX), axes=AX).real * n * m
+    out = torch.empty((planes, n, m), dtype=odt, device=gpu)
+    D.uv_to_image(torch.from_numpy(g).to(gpu), torch.from_numpy(sw).to(gpu), out,
+                  D.fft_work(planes, n, m, gpu), taper=False)
+    assert _rel(out.cpu().numpy(), ref / sw[:, None, None]) < tol
