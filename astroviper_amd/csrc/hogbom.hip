@@ -644,9 +644,24 @@ __global__ __launch_bounds__(256) void k_maximg(const T *__restrict__ img,
   }
 }
 
-__global__ void k_hog_clear(uint32_t *w, int n) {
+// Before a launch: zero the arrivals, the error mark (unless another plane of
+// the call set it: `first` false) and the slots, `n` words in all, and mark the
+// planes' results as not reached: a group that misses an exchange leaves its
+// remaining planes so.  The header's words between are a single plane's result.
+__global__ void k_hog_clear(uint32_t *w, int n, bool first, HogResult *result, int n_planes) {
+  constexpr int kHead = (int)(kHogHeaderBytes / 4);
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) w[i] = 0u;
+  if (i == 0 || (i == 1 && first) || (i >= kHead && i < n)) w[i] = 0u;
+  if (i < n_planes) result[i].reason = -1;
+}
+
+static int launch_hog_clear(void *work, int words, bool first, HogResult *result, int n_planes,
+                            hipStream_t s) {
+  const int n = std::max(words, n_planes);
+  hipLaunchKernelGGL(k_hog_clear, dim3((n + 255) / 256), dim3(256), 0, s, (uint32_t *)work, words,
+                     first, result, n_planes);
+  AV_LAUNCH_CHECK("k_hog_clear");
+  return AV_OK;
 }
 
 // One plane by row bands (any size).
@@ -659,9 +674,8 @@ static int launch_hogbom_bands(const HogRegArgs &A, void *model, void *resid, co
   int groups = std::min(std::min(prop.num_cus * std::max(per_cu, 0), kHogMaxGroups), A.ny);
   if (groups < 1) return fail(AV_ERR_HIP, "av_hogbom_clean: no resident workgroup possible");
   groups = std::min(groups, prop.num_cus);  // one band per CU
-  hipLaunchKernelGGL(k_hog_clear, dim3(1), dim3(64), 0, s, (uint32_t *)work,
-                     (int)(kHogHeaderBytes / 4));
-  AV_LAUNCH_CHECK("k_hog_clear");
+  const int rc = launch_hog_clear(work, (int)(kHogHeaderBytes / 4), result == A.result, result, 1, s);
+  if (rc) return rc;
   T *m = (T *)model, *r = (T *)resid;
   const T *p = (const T *)psf, *k = (const T *)A.mask;
   T tg = (T)A.gain, tt = (T)A.thres, tc = (T)A.cspeedup;
@@ -752,9 +766,7 @@ static int launch_hogbom(HogRegArgs &A, void *work, hipStream_t s) {
   A.slots = (unsigned long long *)((char *)work + kHogHeaderBytes);
   // phase bits 0 in every slot: what no round of the first two expects
   const int words = (int)(kHogHeaderBytes / 4) + L.wgs * L.groups * 8;
-  hipLaunchKernelGGL(k_hog_clear, dim3((words + 255) / 256), dim3(256), 0, s, (uint32_t *)work,
-                     words);
-  AV_LAUNCH_CHECK("k_hog_clear");
+  if ((rc = launch_hog_clear(work, words, true, A.result, A.n_planes, s))) return rc;
   if (L.h == 8) return launch_hogbom_reg<T, 8>(A, s);
   if (L.h == 16) return launch_hogbom_reg<T, 16>(A, s);
   if (L.h == kMost / 2) return launch_hogbom_reg<T, kMost / 2>(A, s);

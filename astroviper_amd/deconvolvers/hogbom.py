@@ -151,7 +151,7 @@ def clean_device(residual: torch.Tensor, psf: torch.Tensor, model: torch.Tensor,
         head = work[:32].cpu().numpy()
         it, px, py, reason = (int(x) for x in head[8:24].view(np.int32))
         maxval = dt(head[24:32].view(np.float64)[0])
-        if reason < 0:
+        if reason < 0 or head[4:8].any():
             raise _lib.AvgridError("av_hogbom_clean: a workgroup did not reach the grid barrier")
         if reason != 1:
             break
@@ -200,8 +200,11 @@ def clean_planes_device(residual: torch.Tensor, psf: torch.Tensor, model: torch.
     _lib.call("av_hogbom_clean_planes", _dev._ptr(model), _dev._ptr(residual), _dev._ptr(psf), n,
               int(planes_per_psf), nx, ny, int(max_iter), float(dt(gain)), float(dt(threshold)),
               _code(dt), _dev._ptr(result), _dev._ptr(work), _dev._stream())
-    head = result.cpu().numpy()
-    if np.any(head[:, 3] < 0):
+    # every plane's record, and the mark of a workgroup that gave up in the
+    # work's header: it need not be one that wrote a record
+    head = torch.cat((result.reshape(-1), work[4:8].view(torch.int32))).cpu().numpy()
+    missed, head = head[-1], head[:-1].reshape(n, 6)
+    if n and (missed or np.any(head[:, 3] < 0)):
         raise _lib.AvgridError("av_hogbom_clean_planes: a workgroup did not reach the exchange")
     return head[:, 0]
 

@@ -368,8 +368,9 @@ int av_hogbom_clean(void *model, void *residual, const void *psf,
  * deconvolution.py:224-287.  model and residual [n_planes][ny][nx]; plane p
  * uses PSF p / planes_per_psf of psf [..][ny][nx].  result: n_planes records
  * of 24 bytes {int32 iterations, x, y of the last peak, reason; double last
- * peak}; reason -1 says that a workgroup did not reach an exchange.  Planes
- * run side by side on the chip. */
+ * peak}; reason -1 says that a workgroup did not reach an exchange, or that the
+ * plane was not begun after one that did not, and the error word of work's
+ * header is then not 0.  Planes run side by side on the chip. */
 int av_hogbom_clean_planes(void *model, void *residual, const void *psf, int32_t n_planes,
                            int32_t planes_per_psf, int32_t nx, int32_t ny, int32_t niter,
                            double gain, double thres, int32_t dtype, void *result, void *work,
