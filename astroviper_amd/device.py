@@ -356,7 +356,8 @@ class GridPlan:
             return vis_out
         mode = ((AV_DEGRID_INCREMENTAL if incremental else 0)
                 | (AV_DEGRID_F32_PRODUCTS if f32_products else 0))
-        call("av_degrid", self._h, _ptr(grid.contiguous()), int(npol_g), _ptr(pol_map),
+        grid = grid.contiguous()  # held until the call is made
+        call("av_degrid", self._h, _ptr(grid), int(npol_g), _ptr(pol_map),
              _ptr(flag), int(n_pol), _ptr(self.cgk), _ptr(vis_out), code, mode, _stream())
         return vis_out
 
@@ -431,7 +432,8 @@ def uv_to_image(grid: torch.Tensor, sumwt: Optional[torch.Tensor], out: torch.Te
     """real(fftshift(N^2 ifft2(ifftshift(grid)))) / taper / sumwt per plane
     into `out` (real), in FP64."""
     n_u, n_v = grid.shape[-2:]
-    call("av_uv_to_image", _ptr(_aligned(grid, 16)), _real_code(grid.dtype),
+    grid = _aligned(grid, 16)  # held until the call is made
+    call("av_uv_to_image", _ptr(grid), _real_code(grid.dtype),
          grid.numel() // (n_u * n_v), n_u, n_v, _ptr(sumwt), int(taper), _ptr(out),
          _real_code(out.dtype), _ptr(work), _stream())
     return out
@@ -442,8 +444,9 @@ def image_to_uv(image: torch.Tensor, out: torch.Tensor, work: torch.Tensor,
     """fftshift(fft2(ifftshift(image / taper))) of a real image into `out`
     (complex), in FP64."""
     n_u, n_v = image.shape[-2:]
-    call("av_image_to_uv", _ptr(_aligned(image, 16)), _real_code(image.dtype),
-         image.numel() // (n_u * n_v), n_u, n_v, int(taper), _ptr(out), _real_code(out.dtype), _ptr(work), _stream())
+    image = _aligned(image, 16)  # held until the call is made
+    call("av_image_to_uv", _ptr(image), _real_code(image.dtype), image.numel() // (n_u * n_v),
+         n_u, n_v, int(taper), _ptr(out), _real_code(out.dtype), _ptr(work), _stream())
     return out
 
 

@@ -1,8 +1,37 @@
 """How the Python layer makes its device calls, without a GPU: the library's
 entry points are replaced, so tensors stay on the CPU."""
+import weakref
+
 import pytest
 
 torch = pytest.importorskip("torch")
+
+
+def test_copies_for_a_call_live_until_it_is_made(monkeypatch):
+    """An operand copied for its alignment or layout is still held when the
+    library is called: freed before, another thread's tensor could take its
+    memory on the same stream."""
+    from astroviper_amd import device as D
+    passed, alive = [], []
+    monkeypatch.setattr(D, "_aligned", lambda t, n: None if t is None else t.clone())
+    monkeypatch.setattr(D, "_ptr", lambda t: None if t is None else passed.append(weakref.ref(t)))
+    monkeypatch.setattr(D, "_stream", lambda: None)
+    monkeypatch.setattr(D, "call", lambda *a: alive.append(all(t() is not None for t in passed)))
+    g = torch.zeros((1, 1, 8, 8), dtype=torch.complex64)
+    x = torch.zeros((1, 1, 8, 8))
+    work = torch.zeros(1, dtype=torch.uint8)
+    D.uv_to_image(g, None, x.clone(), work)
+    passed.clear()
+    D.image_to_uv(x, g.clone(), work)
+    passed.clear()
+    plan = object.__new__(D.GridPlan)
+    plan.n_rows, plan.n_chan, plan.row_chan, plan._h = 4, 1, None, None
+    plan.device, plan.cgk = torch.device("cpu"), torch.zeros(3)
+    plan.degrid(g.transpose(-1, -2), torch.zeros((4, 1), dtype=torch.bool))
+    passed.clear()
+    plan.n_img_chan, plan.n_u, plan.n_v = 1, 8, 8
+    plan.grid(torch.zeros((4, 1), dtype=torch.complex64), torch.ones((4, 1)))
+    assert alive == [True] * 4
 
 
 def _fake_clean(monkeypatch, H, planes):
