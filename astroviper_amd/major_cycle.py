@@ -36,6 +36,16 @@ from .deconvolvers import hogbom as H
 _SIGNS = {}
 
 
+def _values_only(t: torch.Tensor) -> bool:
+    """Whether a kernel on the tensor's memory does all that torch's own
+    operations on it would: device memory, no gradient to record (backward or
+    forward mode), no function transform, no tensor of another type."""
+    return (t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter)
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+
+
 def model_to_uv(model: torch.Tensor, cdt: torch.dtype) -> torch.Tensor:
     """fftshift(fft2(ifftshift(model))) over the last two axes, in the
     complex dtype `cdt`: fft_lm_to_uv as predict_model_visibilities applies
@@ -52,10 +62,12 @@ def model_to_uv(model: torch.Tensor, cdt: torch.dtype) -> torch.Tensor:
     prime factors beyond 5 take av_image_to_uv, two passes that do everything;
     else the flipped image is formed in the real dtype in one pass, transformed,
     and av_hermitian_expand writes the whole spectrum from the half
-    (F[-k] = conj(F[k])) with the output flip, in one pass."""
+    (F[-k] = conj(F[k])) with the output flip, in one pass.  A model that is
+    more than its values (recorded for a gradient, transformed, on the host)
+    keeps torch's operations where its axes are no multiples of 4."""
     ny, nx = model.shape[-2:]
     ax = (-2, -1)
-    if not model.is_complex() and cdt == torch.complex128:
+    if not model.is_complex() and cdt == torch.complex128 and _values_only(model):
         work = D.fft_work(model.numel() // max(1, ny * nx), ny, nx, model.device)
         if work is not None:
             if model.dtype not in (torch.float32, torch.float64):

@@ -2,9 +2,12 @@
 entry points are replaced, so tensors stay on the CPU."""
 import weakref
 
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
+
+AX = (-2, -1)
 
 
 def test_copies_for_a_call_live_until_it_is_made(monkeypatch):
@@ -32,6 +35,23 @@ def test_copies_for_a_call_live_until_it_is_made(monkeypatch):
     plan.n_img_chan, plan.n_u, plan.n_v = 1, 8, 8
     plan.grid(torch.zeros((4, 1), dtype=torch.complex64), torch.ones((4, 1)))
     assert alive == [True] * 4
+
+
+@pytest.mark.parametrize("shape", [(2, 18, 30), (3, 2, 50, 36), (1, 6, 10)])
+def test_model_to_uv_on_the_host(shape):
+    """Even axes that are no multiples of 4 are transformed by torch wherever
+    the model lies, with its gradient, as any tensor function."""
+    from astroviper_amd.major_cycle import model_to_uv
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal(shape)
+    ref = np.fft.fftshift(np.fft.fft2(np.fft.ifftshift(x, axes=AX), axes=AX), axes=AX)
+    t = torch.from_numpy(x).requires_grad_(True)
+    uv = model_to_uv(t, torch.complex128)
+    # two FP64 transforms of a few hundred points: a few roundings of the largest
+    np.testing.assert_allclose(uv.detach().numpy(), ref, rtol=0, atol=1e-13 * np.abs(ref).max())
+    torch.view_as_real(uv).square().sum().backward()
+    grad = 2 * shape[-2] * shape[-1] * x
+    np.testing.assert_allclose(t.grad.numpy(), grad, rtol=0, atol=1e-13 * np.abs(grad).max())
 
 
 def _fake_clean(monkeypatch, H, planes):

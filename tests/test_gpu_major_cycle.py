@@ -161,3 +161,24 @@ def test_deconvolve_of_strided_images(gpu):
             assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
             np.testing.assert_array_equal(got[2], ref[2])
     im.close()
+
+
+def test_model_to_uv_of_a_recorded_model(gpu):
+    """Axes that are even but no multiples of 4 keep torch's gradient: that of
+    sum |F|^2 is 2 N^2 x."""
+    from astroviper_amd.major_cycle import model_to_uv
+    x = torch.randn((2, 18, 50), dtype=torch.float64, device=gpu)
+    t = x.clone().requires_grad_(True)
+    uv = model_to_uv(t, torch.complex128)
+    torch.view_as_real(uv).square().sum().backward()
+    assert rel(t.grad.cpu().numpy(), 2 * 18 * 50 * x.cpu().numpy()) < 1e-13
+    assert rel(model_to_uv(x, torch.complex128).cpu().numpy(), uv.detach().cpu().numpy()) < 1e-13
+    with torch.no_grad():
+        assert not model_to_uv(t, torch.complex128).requires_grad
+    # the transform is linear: its derivative along v is the transform of v
+    v = torch.randn_like(x)
+    _, d = torch.func.jvp(lambda a: model_to_uv(a, torch.complex128), (x,), (v,))
+    ref = model_to_uv(v, torch.complex128).cpu().numpy()
+    assert rel(d.cpu().numpy(), ref) < 1e-13
+    many = torch.func.vmap(lambda a: model_to_uv(a, torch.complex128))(v.reshape(2, 1, 18, 50))
+    assert rel(many.reshape(v.shape).cpu().numpy(), ref) < 1e-13
