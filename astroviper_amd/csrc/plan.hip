@@ -1060,6 +1060,18 @@ static int32_t default_unit_cap(int64_t n_items) {
   return cap;
 }
 
+// Time steps that a chunk spans before its rows are visited baseline by
+// baseline.  Two make runs of two records, and a chunk's positions outside its
+// rows are at most half of all; in row order a wavefront's records go to as
+// many bins as it has lanes.  Cubes of 64 antennas x 16 channels, binning in row
+// order and so: 4.7 steps 341 -> 253 us, 3.1 250 -> 198, 2.3 (FP64) 194 -> 166,
+// 15.6 on 2048^2 planes 1248 -> 797; continuum of 4 channels x 2.9 steps 1254 ->
+// 843.  Where a chunk takes every channel of a row, many channels fill a
+// wavefront already (48 channels x 2.5 steps 1130 -> 1200, 64 x 2 565 -> 640; 16
+// x 4 783 -> 661).
+constexpr int64_t kOrderSteps = 2, kOrderStepsWide = 16;
+constexpr int kOrderChans = 32;
+
 // Rows of a chunk.  Every chunk is a workgroup of the two binning passes:
 // kChunkTarget of them in all keep the chip busy, but a chunk also reads and
 // writes a word per tile in each of four passes, so it has at least half a
@@ -1387,9 +1399,10 @@ int av_plan_set_row_order(av_plan *plan, int32_t n_baseline) {
   PlanDev &d = plan->d;
   if (n_baseline < 1 || (d.n_rows > 0 && d.n_rows % n_baseline != 0))
     return fail(AV_ERR_INVALID, "av_plan_set_row_order: n_baseline must be >= 1 and divide n_rows");
-  // a chunk is visited baseline by baseline only when it spans at least 16
-  // time steps; otherwise the runs per bin stay short and row order is kept
-  d.order_nb = (n_baseline > 1 && (int64_t)n_baseline * 16 <= d.rows_per_chunk) ? n_baseline : 1;
+  // a chunk is visited baseline by baseline where it spans a few time steps (see
+  // kOrderSteps)
+  const int64_t steps = d.chunk_all && d.n_chan >= kOrderChans ? kOrderStepsWide : kOrderSteps;
+  d.order_nb = (n_baseline > 1 && n_baseline * steps <= d.rows_per_chunk) ? n_baseline : 1;
   return AV_OK;
 }
 

@@ -211,3 +211,21 @@ def test_compensated_sums_of_neighbouring_split_bins(gpu, oracle, cap, per_tile,
     g, sw = plan.grid(None, dev(w), grid=g, sumwt=sw, psf=True, accumulate=True, compensated=True)
     assert _rel(g.cpu().numpy(), 2 * gref) < 16 * 2.0 ** -24
     plan.close()
+
+
+@pytest.mark.parametrize("nt,nb,nchan,cube", [
+    (5, 512, 3, True),     # chunks of 1024 rows: two time steps, then a part
+    (5, 513, 3, True),     # one row fewer than two
+    (40, 171, 31, False),  # all channels of 64-row chunks, rows in order
+    (3, 30, 31, False),    # two steps and a part, 31 channels
+    (3, 30, 32, False),    # as many channels as keep row order
+])
+def test_binning_of_few_time_steps_a_chunk(gpu, oracle, nt, nb, nchan, cube):
+    n_uv = (96, 80)
+    uvw, freq, vis, w, flag, cell = _samples(nt, nb, nchan, 1, n_uv, nb + nchan)
+    gref, swref = oracle.standard_grid(vis, uvw, np.where(flag, 0.0, w), freq, n_uv, cell,
+                                       chan_mode="cube" if cube else "continuum")
+    g, sw, m, st = _run(gpu, uvw, freq, vis, w, flag, n_uv, cell, cube, nb)
+    mref = oracle.degrid(uvw, flag, freq, gref, cell)
+    assert _rel(g, gref) < 1e-12 and _rel(sw, swref) < 1e-12
+    assert _rel(m.reshape(mref.shape), mref) < 1e-12
