@@ -213,15 +213,16 @@ def test_compensated_sums_of_neighbouring_split_bins(gpu, oracle, cap, per_tile,
     plan.close()
 
 
-@pytest.mark.parametrize("nt,nb,nchan,cube", [
-    (5, 512, 3, True),     # chunks of 1024 rows: two time steps, then a part
-    (5, 513, 3, True),     # one row fewer than two
-    (40, 171, 31, False),  # all channels of 64-row chunks, rows in order
-    (3, 30, 31, False),    # two steps and a part, 31 channels
-    (3, 30, 32, False),    # as many channels as keep row order
+@pytest.mark.parametrize("nt,nb,nchan,n,cube", [
+    (5, 512, 3, 80, True),      # chunks of 1024 rows: rows in order
+    (5, 1536, 2, 1040, True),   # chunks of 3072 rows: two time steps, then a part
+    (5, 1537, 2, 1040, True),   # one row fewer than two
+    (9, 33, 31, 80, False),     # all channels of 66 rows and more, 31 and 32
+    (9, 33, 32, 80, False),
+    (40, 32, 31, 528, False),
 ])
-def test_binning_of_few_time_steps_a_chunk(gpu, oracle, nt, nb, nchan, cube):
-    n_uv = (96, 80)
+def test_binning_of_few_time_steps_a_chunk(gpu, oracle, nt, nb, nchan, n, cube):
+    n_uv = (n + 16, n)
     uvw, freq, vis, w, flag, cell = _samples(nt, nb, nchan, 1, n_uv, nb + nchan)
     gref, swref = oracle.standard_grid(vis, uvw, np.where(flag, 0.0, w), freq, n_uv, cell,
                                        chan_mode="cube" if cube else "continuum")
