@@ -159,7 +159,8 @@ struct PlanDev {
   int32_t n_chan, n_img_chan, n_u, n_v;
   double cell_u, cell_v;
   double dscale_u, dscale_v, doff_u, doff_v;  // degrid pixel transform
-  int32_t support, ov, tile_u, tile_v, geometry, unit_cap;
+  int32_t support, ov, tile_u, tile_v, geometry;
+  int32_t unit_cap, dunit_cap;  // records of a grid unit, of a degrid or pair unit
   int32_t conjugate;  // AV_GEOM_CONJUGATE: samples at their conjugate centres
   // x / tile as __umulhi(x, tile_*_mul), exact for 0 <= x < 2^24 (tiles <= 128)
   uint32_t tile_u_mul, tile_v_mul;

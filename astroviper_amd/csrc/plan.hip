@@ -784,11 +784,11 @@ __device__ inline void block_scan_n(uint32_t (&v)[N], uint32_t (&total)[N], uint
 }
 
 __device__ inline void bin_values(const PlanDev &P, int64_t b, uint32_t (&v)[3]) {
-  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t cap = (uint32_t)P.unit_cap, dcap = (uint32_t)P.dunit_cap;
   const uint32_t na = P.cnt_all[b], np = P.cnt_prim[b];
   v[0] = na;
   v[1] = na == 0 ? 1u : (na + cap - 1) / cap;
-  v[2] = (np + cap - 1) / cap;
+  v[2] = (np + dcap - 1) / dcap;
 }
 
 __device__ inline uint32_t pair_value(const PlanDev &P, int64_t p) {
@@ -796,7 +796,7 @@ __device__ inline uint32_t pair_value(const PlanDev &P, int64_t p) {
   bool has1;
   uint32_t n;
   pair_bins(P, p, b0, b1, has1, n);
-  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t cap = (uint32_t)P.dunit_cap;
   return (n + cap - 1) / cap;
 }
 
@@ -804,7 +804,7 @@ __device__ inline uint32_t pair_value(const PlanDev &P, int64_t p) {
 // `carry` records, grid units and degrid units (updated).
 __device__ inline void index_bins(const PlanDev &P, int64_t b0, int64_t b1, uint32_t (&carry)[3],
                                   uint32_t *sh) {
-  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t cap = (uint32_t)P.unit_cap, dcap = (uint32_t)P.dunit_cap;
   for (int64_t base = b0; base < b1; base += blockDim.x) {
     const int64_t b = base + threadIdx.x;
     const bool on = b < b1;
@@ -831,14 +831,14 @@ __device__ inline void index_bins(const PlanDev &P, int64_t b0, int64_t b1, uint
       P.gunits[v[1] + k] = make_uint4((uint32_t)b, v[0] + k * cap, cnt, fl);
     }
     for (uint32_t k = 0; k < n[2]; ++k)
-      P.dunits[v[2] + k] = make_uint4((uint32_t)b, v[0] + k * cap, min(cap, np - k * cap), 0u);
+      P.dunits[v[2] + k] = make_uint4((uint32_t)b, v[0] + k * dcap, min(dcap, np - k * dcap), 0u);
   }
 }
 
 // Pair units of pairs [p0, p1), preceded by `carry` units (updated).
 __device__ inline void index_pairs(const PlanDev &P, int64_t p0, int64_t p1, uint32_t &carry,
                                    uint32_t *sh) {
-  const uint32_t cap = (uint32_t)P.unit_cap;
+  const uint32_t cap = (uint32_t)P.dunit_cap;
   for (int64_t base = p0; base < p1; base += blockDim.x) {
     const int64_t p = base + threadIdx.x;
     const bool on = p < p1;
@@ -1060,6 +1060,19 @@ static int32_t default_unit_cap(int64_t n_items) {
   return cap;
 }
 
+// A degrid unit loads its tile's cells before its first record, where a grid
+// unit starts from zeros, so short ones cost it more: caps of four grid units
+// where a plan has four image channels or more, whose dense bins share the chip,
+// the grid unit's own where one plane holds them all.  Degridding alone, us at
+// caps of 256, 512, 1024, 2048, 4096 and 8192 (grid caps of 256 and 512): 1.9 M
+// samples x 4 polarisations on 8 planes of 1024^2 159, 145, 140, 146, 145 and
+// 146, on one plane 128, 116, 122, 141, 167 and 250; 6.5 M on 8 planes 469, 419,
+// 403, 391, 403 and 432, on two 438, 389, 371, 380, 407 and 503, on one 396, 347,
+// 332, 342, 373 and 442.
+static int32_t default_dunit_cap(int64_t n_items, int32_t n_img_chan) {
+  return default_unit_cap(n_items * std::min(n_img_chan, 4));
+}
+
 // Time steps that a chunk spans before its rows are visited baseline by
 // baseline.  Two make runs of two records, and a chunk's positions outside its
 // rows are at most half of all; in row order a wavefront's records go to as
@@ -1129,10 +1142,14 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   if (conjugate && geometry != AV_GEOM_REFERENCE)
     return fail(AV_ERR_INVALID, "av_plan_create: AV_GEOM_CONJUGATE needs AV_GEOM_REFERENCE");
   int64_t n_items = row_channels ? n_rows : n_rows * (int64_t)n_chan;
-  if (unit_cap == 0) unit_cap = compact ? 8192 : default_unit_cap(n_items);
-  if (unit_cap < 64) return fail(AV_ERR_INVALID, "av_plan_create: unit_cap < 64");
   if (n_items > ((int64_t)1 << 32) / 5 - 1)
     return fail(AV_ERR_UNSUPPORTED, "av_plan_create: more than 858993458 samples per plan");
+  int32_t dunit_cap = unit_cap;
+  if (unit_cap == 0) {
+    unit_cap = compact ? 8192 : default_unit_cap(n_items);
+    dunit_cap = compact ? 8192 : default_dunit_cap(n_items, n_img_chan);
+  }
+  if (unit_cap < 64) return fail(AV_ERR_INVALID, "av_plan_create: unit_cap < 64");
 
   PlanDev &d = p->d;
   d.n_rows = n_rows;
@@ -1157,6 +1174,7 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.conjugate = conjugate ? 1 : 0;
   d.row_channels = row_channels;
   d.unit_cap = unit_cap;
+  d.dunit_cap = dunit_cap;
   d.ntu = (n_u + tile_u - 1) / tile_u;
   d.ntv = (n_v + tile_v - 1) / tile_v;
   d.n_bins = (int64_t)d.ntu * d.ntv * n_img_chan;
@@ -1167,10 +1185,10 @@ int plan_layout(int64_t n_rows, int32_t n_chan, int32_t n_img_chan, int32_t n_u,
   d.max_records = 5 * n_items;
   d.max_gunits = d.n_bins + d.max_records / unit_cap + 1;
   // a sample has at most two primary records (grid + separate degrid)
-  d.max_dunits = d.n_bins + 2 * n_items / unit_cap + 1;
+  d.max_dunits = d.n_bins + 2 * n_items / dunit_cap + 1;
   const bool pairs = tile_u == 16 && tile_v == 16 && support <= 7;
   d.n_pairs = pairs ? (int64_t)d.ntu * ((d.ntv + 1) / 2) * n_img_chan : 0;
-  d.max_punits = pairs ? d.n_pairs + 2 * n_items / unit_cap + 1 : 0;
+  d.max_punits = pairs ? d.n_pairs + 2 * n_items / dunit_cap + 1 : 0;
   d.row_chan = nullptr;
   d.order_nb = 1;
   d.uvw = nullptr;

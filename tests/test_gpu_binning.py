@@ -230,3 +230,30 @@ def test_binning_of_few_time_steps_a_chunk(gpu, oracle, nt, nb, nchan, n, cube):
     mref = oracle.degrid(uvw, flag, freq, gref, cell)
     assert _rel(g, gref) < 1e-12 and _rel(sw, swref) < 1e-12
     assert _rel(m.reshape(mref.shape), mref) < 1e-12
+
+
+@pytest.mark.parametrize("nchan", [1, 2, 4])
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_degrid_units_longer_than_grid_units(gpu, nchan, prec):
+    """Plans of samples enough for degrid caps of two and four grid caps: a
+    sample's sum does not depend on its unit, so one cap for both gives the same
+    bits, on bins of many units and of one."""
+    from astroviper_amd.device import GridPlan
+    cdt = torch.complex64 if prec == "fp32" else torch.complex128
+    n, nb, nt = 112, 350, 1 + 1_300_000 // (350 * nchan)
+    uvw, freq, _, _, _, cell = _samples(nt, nb, nchan, 1, (n, n), nchan, spread=0.3)
+    gen = torch.Generator(device=gpu).manual_seed(nchan)
+    grid = torch.randn((nchan, 2, n, n), generator=gen, device=gpu, dtype=cdt)
+    out, units = [], []
+    for cap in (0, 8192, 64):
+        plan = GridPlan(nt * nb, nchan, nchan, (n, n), cell, unit_cap=cap, device=gpu,
+                        n_baseline=nb)
+        plan.set_uvw(torch.from_numpy(uvw.reshape(-1, 3)).to(gpu), torch.from_numpy(freq).to(gpu))
+        out.append(plan.degrid(grid))
+        units.append((plan.stats()["grid_units"], plan.stats()["degrid_units"]))
+        plan.close()
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    assert float(out[0].abs().max()) > 0
+    # 256 records a grid unit; as many, two and four times as many a degrid unit
+    ratio = units[0][0] / units[0][1]
+    assert ratio > {1: 1.0, 2: 1.8, 4: 3.0}[nchan]
