@@ -564,12 +564,32 @@ constexpr int grid_mfma_min_blocks() {
 // wavefronts to a SIMD; eight share a table where there are units enough for
 // every compute unit (twice over): 643 -> 585 us for 4.8 M samples x 2
 // polarisations on 16 planes of 1024^2, but 36 -> 42 us for a snapshot's 256
-// tiles, whose workgroups of eight leave most of the chip idle.
+// tiles, whose workgroups of eight leave most of the chip idle.  Four
+// polarisations need 150 registers, three wavefronts to a SIMD, which eight per
+// workgroup would not all be: 13 M samples on 64 planes of 2048^2 take 5.80 ms in
+// workgroups of four, 6.55 of eight.  The kernel is compiled for eight all the
+// same: bounded for four alone it spreads to 202 registers and takes 6.94.
 constexpr int kGridWideWaves = 8;
 constexpr int64_t kGridWideUnits = 4096;
 template <typename R>
 constexpr int grid_mfma_max_waves() {
   return sizeof(R) == 8 ? kGridWideWaves : kGridMaxWaves;
+}
+template <typename R, int NPOL>
+constexpr bool grid_mfma_wide() {
+  return sizeof(R) == 8 && NPOL <= 2;
+}
+
+// Matrix-core steps of four records unrolled together.  Each waits for two LDS
+// reads in turn (the record's table bases, then its weights), which one step
+// after another left unhidden at three wavefronts per SIMD (FP64, two
+// polarisations: 755 us, four at a time 643, two 684, eight 653; see
+// kGridWideWaves).  Four FP64 polarisations have eight products a step to hide
+// them with: one step at a time 1285 us for 6.5 M samples on 16 planes of 1024^2,
+// two 1316, four 1329.
+template <typename R, int NPOL>
+constexpr int grid_mfma_steps() {
+  return sizeof(R) == 8 && NPOL == 4 ? 1 : 4;
 }
 
 template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF>
@@ -767,17 +787,15 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
     fetch_raw<R, NPOL>(raw1, r1.x, vis, weight, flag, psf, adjoint);
     const uint2 r2 = load_record(P, base + 128 + lane, end);
     wave_lds_sync();
-    // ---- four records per matrix-core step, four steps at a time: each
-    // waits for two LDS reads in turn (the record's table bases, then its
-    // weights), which one step after another left unhidden at three
-    // wavefronts per SIMD (FP64: 755 us, four at a time 643, two 684, eight
-    // 653; see kGridWideWaves).  Steps past the last record add staged zeros.
+    // ---- four records per matrix-core step, several steps at a time; those
+    // past the last record add staged zeros
     const int nst = (int)min((uint32_t)64, end - base);
     const int li_nw = li * L.nw;
-    for (int s16 = 0; s16 < nst; s16 += 16)
+    constexpr int kSteps = 4 * grid_mfma_steps<R, NPOL>();
+    for (int s0 = 0; s0 < nst; s0 += kSteps)
 #pragma unroll
-    for (int s4 = 0; s4 < 16; s4 += 4) {
-      const int rec = s16 + s4 + lk;
+    for (int s4 = 0; s4 < kSteps; s4 += 4) {
+      const int rec = s0 + s4 + lk;
       const uint32_t tb = st_geo[rec];
       const uint32_t tbu = tb & 0xFFFFu, tbv = tb >> 16;
       R a[MB], wv[VB];
@@ -1049,7 +1067,7 @@ static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   const MfmaLds L = mfma_lds_layout<R, NPOL>(d.ov, d.support, 16 * (MB > VB ? MB : VB));
   int nw = kGridMaxWaves;
-  if constexpr (grid_mfma_max_waves<R>() > kGridMaxWaves) {
+  if constexpr (grid_mfma_wide<R, NPOL>()) {
     if (d.max_gunits >= kGridWideUnits &&
         (size_t)(L.st_d + kGridWideWaves * L.wave_bytes) <= prop.lds_per_block)
       nw = kGridWideWaves;
