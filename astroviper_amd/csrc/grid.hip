@@ -18,6 +18,7 @@
 // that a pre-pass zeroed.  Sums of weights are FP64: each unit writes its
 // partial sums and a reduction pass adds them per plane.
 #include <algorithm>
+#include <type_traits>
 
 #include "tile_common.h"
 
@@ -509,11 +510,10 @@ __device__ inline void copy_wtab_padded(R *w, const MfmaLds &L, const PlanDev &P
   }
 }
 
-// LDS in which a compensated group's wavefronts add their tiles in FP64, and
-// the size of a split bin's FP64 slot.
-template <int NPOL, int MB, int VB, bool COMP>
-__host__ __device__ constexpr int mfma_comb_bytes() {
-  return COMP ? MB * 2 * NPOL * VB * 4 * 64 * (int)sizeof(double) : 0;
+// The size of a split bin's FP64 slot.
+template <int NPOL, int MB, int VB>
+__host__ __device__ constexpr int comp_slot_bytes() {
+  return MB * 2 * NPOL * VB * 4 * 64 * (int)sizeof(double);
 }
 
 // A wavefront's tile to the grid: lane l holds rows MfmaOp::row(l / 16, r),
@@ -552,11 +552,18 @@ __device__ inline void store_tile(const PlanDev &P,
 }
 
 // Workgroups per CU the FP32 kernels with up to 8 result blocks are compiled
-// for: six (80 registers, no spills; a 16 x 16 tile's workgroup needs 26 KB
-// of LDS).  Other variants keep the compiler's choice.
-template <typename R, int NPOL, int MB, int VB, bool COMP>
+// for: six with up to 4 (80 registers, no spills; a 16 x 16 tile's workgroup
+// needs 26 KB of LDS), five with 8 (96; at six, which four polarisations' loads do
+// not fit into without being serialised, 1.9 M samples on 8 planes of 1024^2 take
+// 438 us, at five 277).  Compensated sums, whose pairs triple the result blocks:
+// six and five without TEAMS, five and four with.  Other variants keep the
+// compiler's choice.
+template <typename R, int NPOL, int MB, int VB, bool COMP, bool TEAMS>
 constexpr int grid_mfma_min_blocks() {
-  return (sizeof(R) == 4 && !COMP && MB * 2 * NPOL * VB <= 8) ? 6 : 1;
+  constexpr int kBlocks = MB * 2 * NPOL * VB;
+  if (sizeof(R) != 4 || kBlocks > 8) return 1;
+  if (COMP) return (kBlocks <= 2 ? 6 : kBlocks <= 4 ? 5 : 2) - (TEAMS ? 1 : 0);
+  return kBlocks <= 4 ? 6 : 5;
 }
 
 // Wavefronts of a workgroup, at most.  An FP64 weight table takes 33 KB of LDS
@@ -592,22 +599,21 @@ constexpr int grid_mfma_steps() {
   return sizeof(R) == 8 && NPOL == 4 ? 1 : 4;
 }
 
-template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF>
-__global__ __launch_bounds__(64 * grid_mfma_max_waves<R>(),
-                             (grid_mfma_min_blocks<R, NPOL, MB, VB, COMP>()))
-void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
-                                                            const R *__restrict__ weight,
-                                                            const uint8_t *__restrict__ flag,
-                                                            const double *__restrict__ cgk,
-                                                            R *__restrict__ grid, int mode) {
+// Unit u by its wavefront, or (TEAMS) the compensated group that it leads: by one
+// wavefront, or by the whole workgroup (`team`).
+template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF, bool TEAMS>
+__device__ __forceinline__ void grid_mfma_unit(const PlanDev &P, const MfmaLds &L, char *smem,
+                                               const R *__restrict__ vis,
+                                               const R *__restrict__ weight,
+                                               const uint8_t *__restrict__ flag,
+                                               R *__restrict__ grid, int mode, uint32_t u,
+                                               bool team) {
   using MO = MfmaOp<R>;
   using MV = typename MO::V;
   constexpr int C = 2 * NPOL;
-  extern __shared__ __align__(16) char smem[];
-  const int S = P.support, sc = S / 2, ov = P.ov;
-  const MfmaLds L = mfma_lds_layout<R, NPOL>(ov, S, 16 * (MB > VB ? MB : VB));
-  R *tab = (R *)(smem + L.tab);
-  double *nrm = (double *)(smem + L.nrm);
+  const int sc = P.support / 2;
+  const R *tab = (const R *)(smem + L.tab);
+  const double *nrm = (const double *)(smem + L.nrm);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   char *wbase = smem + L.st_d + wave * L.wave_bytes;
   R *st_d = (R *)wbase;                           // [record][C]
@@ -618,22 +624,7 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
   constexpr bool psf = PSF;  // PSF data are real: the imaginary blocks are skipped
   const bool adjoint = (mode & AV_GRID_ADJOINT) != 0;
   const bool accumulate = (mode & AV_GRID_ACCUMULATE) != 0;
-  const int half = ov / 2 + 2;
-
-  const uint32_t n_units = P.gunit_start[P.n_bins];
-  // 16 workgroups of 4 units: the 64 channels of a tile under one L2
-  // (compensated: a workgroup per unit, that of a group's first unit sums the
-  // whole group)
-  const uint32_t units_per_wg = COMP ? 1 : blockDim.x / 64;
-  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup * kGridMaxWaves / units_per_wg);
-  if (blk * units_per_wg >= n_units) return;  // whole workgroup idle
-  copy_wtab_padded(tab, L, P);
-  for (int i = tid; i < L.nnrm; i += blockDim.x) nrm[i] = P.nrm[i];
-  __syncthreads();  // the only workgroup barrier: tables ready
-  // the same for every lane: scalar registers for the unit and its bounds
-  uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane(
-      (int)(COMP ? blk : blk * units_per_wg + wave));
-  if (u >= n_units) return;
+  const int half = P.ov / 2 + 2;
 
   const int Tu = 16 * MB, Tv = 16 * VB;
   const uint4 unit = P.gunits[u];
@@ -641,10 +632,7 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
   uint32_t first = unit.y, cnt = unit.z;
   bool multi = (unit.w & kUnitMulti) != 0;
   uint32_t n_in = 1;
-  if (COMP) {
-    if (!comp_group(P, b, first, n_in, cnt, multi)) return;
-    if (wave >= (int)n_in && n_in == 1) return;
-  }
+  if (TEAMS) comp_group(P, b, first, n_in, cnt, multi);
   uint32_t tile;
   int ic;
   bin_parts(P, (uint32_t)b, tile, ic);
@@ -704,10 +692,10 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
             acc[m][c][vb][r] = reset ? (R)0 : t + ccmp[k];
           }
   };
-  // wavefronts of a compensated group take its units in turn
-  const uint32_t gend = first + cnt, lead = u;
-  for (uint32_t w = COMP ? (uint32_t)wave : 0u; w < n_in; w += kGridMaxWaves) {
-  if (COMP) {
+  // a compensated group's units, by one wavefront or by all in turn
+  const uint32_t gend = first + cnt, lead = u, step = team ? kGridMaxWaves : 1;
+  for (uint32_t w = team ? (uint32_t)wave : 0u; w < n_in; w += step) {
+  if (TEAMS) {
     u = lead + w;
     first = unit.y + w * (uint32_t)P.unit_cap;
   }
@@ -715,7 +703,7 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
 #pragma unroll
   for (int p = 0; p < NPOL; ++p) sw[p] = 0.0;
 
-  const uint32_t end = COMP ? min(gend, first + (uint32_t)P.unit_cap) : gend;
+  const uint32_t end = TEAMS ? min(gend, first + (uint32_t)P.unit_cap) : gend;
   uint2 r0 = load_record(P, first + lane, end), r1 = load_record(P, first + 64 + lane, end);
   RawSample<R, NPOL> raw0;
   fetch_raw<R, NPOL>(raw0, r0.x, vis, weight, flag, psf, adjoint);
@@ -837,53 +825,146 @@ void k_grid_mfma(PlanDev P, const R *__restrict__ vis,
     for (int off = 32; off >= 1; off >>= 1) sv += __shfl_xor(sv, off);
     if (lane == 0) P.upart[(size_t)u * 4 + p] = sv;
   }
-  if (COMP) fold(w + kGridMaxWaves < n_in);
+  if (COMP) fold(w + step < n_in);
   }
-  if constexpr (COMP) {
-    if (n_in > 1) {
-      // the wavefronts' (sum, compensation) pairs, added in FP64 through LDS
-      double *comb = (double *)(smem + L.total);  // [kNc][64]
+  if (!TEAMS || (!team && !multi)) {
+    // ---- flush: lane holds rows MO::row(lane/16, r), column lane%16 of every block
+    store_tile<R, NPOL, MB, VB>(P, acc, gplane, u0, v0, multi, accumulate);
+    return;
+  }
+  if constexpr (TEAMS) {
+    // a bin of several groups goes into its FP64 slot, which k_comp_slots rounds
+    // to the grid once, others straight into the grid; value by value, as whole
+    // tiles of FP64 values would take the registers of two more wavefronts
+    double *slots = multi ? comp_slots(P, comp_slot_bytes<NPOL, MB, VB>()) : nullptr;
+    double *slot =
+        slots ? slots + (size_t)(P.bin_start[b] / kCompGroupRecords) * (kNc * 64) + lane : nullptr;
+    const auto flush = [&](int k, double x) {
+      if (slot) {
+        if (x != 0.0) unsafeAtomicAdd(slot + k * 64, x);
+        return;
+      }
+      const int m = k / (C * VB * 4), c = k / (VB * 4) % C, vb = k / 4 % VB, r = k % 4;
+      const int gu = u0 + 16 * m + MO::row(lk, r), gv = v0 + 16 * vb + li;
+      if (gu >= P.n_u || gv >= P.n_v) return;
+      R *dst = gplane + (c / 2) * pstride + ((size_t)gu * P.n_v + gv) * 2 + (c & 1);
+      if (multi)
+        atomicAdd(dst, (R)x);
+      else
+        *dst = accumulate ? *dst + (R)x : (R)x;
+    };
+    if (team) {
+      // the wavefronts' (sum, compensation) pairs, added in FP64 through LDS: in
+      // the wavefronts' staging areas, which are free by then, a few values at a
+      // time
+      constexpr int kPart = 4 * NPOL;
+      static_assert(kNc % kPart == 0, "whole parts");
+      static_assert(kPart * 64 * sizeof(double) <= kGridMaxWaves * 64 * (C * sizeof(R) + 4),
+                    "a part fits the staging areas");
+      double *comb = (double *)(smem + L.st_d);  // [kPart][64]
       const int nwv = min(kGridMaxWaves, (int)n_in);
-      for (int w = 0; w < nwv; ++w) {
-        if (wave == w) {
 #pragma unroll
-          for (int k = 0; k < kNc; ++k) {
-            const double x = (double)csum[k] + (double)ccmp[k];
-            comb[k * 64 + lane] = w == 0 ? x : comb[k * 64 + lane] + x;
+      for (int k0 = 0; k0 < kNc; k0 += kPart) {
+        for (int w = 0; w < nwv; ++w) {
+          __syncthreads();
+          if (wave == w) {
+#pragma unroll
+            for (int k = 0; k < kPart; ++k) {
+              // opaque, or the compiler forms all sums ahead of the loop
+              R sum = csum[k0 + k];
+              asm volatile("" : "+v"(sum));
+              const double x = (double)sum + (double)ccmp[k0 + k];
+              comb[k * 64 + lane] = w == 0 ? x : comb[k * 64 + lane] + x;
+            }
           }
         }
         __syncthreads();
+#pragma unroll 1
+        for (int k = wave; k < kPart; k += kGridMaxWaves) flush(k0 + k, comb[k * 64 + lane]);
       }
-      if (wave != 0) return;
-#pragma unroll
-      for (int m = 0; m < MB; ++m)
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-          for (int vb = 0; vb < VB; ++vb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              acc[m][c][vb][r] = (R)comb[(((m * C + c) * VB + vb) * 4 + r) * 64 + lane];
-    }
-  }
-
-  // ---- flush: lane holds rows MO::row(lane/16, r), column lane%16 of every block
-  if constexpr (COMP) {
-    // a bin of several groups: into its FP64 slot, which k_comp_slots rounds
-    // to the grid once
-    double *slots = multi ? comp_slots(P, mfma_comb_bytes<NPOL, MB, VB, true>()) : nullptr;
-    if (slots) {
-      const double *comb = (const double *)(smem + L.total);
-      double *slot = slots + (size_t)(P.bin_start[b] / kCompGroupRecords) * (kNc * 64);
+      __syncthreads();  // the staging areas are the wavefronts' again
+    } else {
 #pragma unroll
       for (int k = 0; k < kNc; ++k) {
-        const double x = n_in > 1 ? comb[k * 64 + lane] : (double)csum[k] + (double)ccmp[k];
-        if (x != 0.0) unsafeAtomicAdd(slot + k * 64 + lane, x);
+        flush(k, (double)csum[k] + (double)ccmp[k]);
       }
-      return;
     }
   }
-  store_tile<R, NPOL, MB, VB>(P, acc, gplane, u0, v0, multi, accumulate);
+}
+
+// Compensated sums run by groups of a bin's units (comp_group).  With TEAMS a
+// workgroup looks at `share` units (0: at every gridDim.x-th unit of a split bin):
+// groups of up to most_alone units, as most bins of a cube are, go to a wavefront
+// each, and the whole workgroup takes the longer ones that its units lead.
+// Without, split bins are left to another launch.  A workgroup per unit, most of
+// them for one wavefront, took 806 us for 1.9 M samples x 4 polarisations on 8
+// planes of 1024^2 where this takes 518, 378 with two polarisations where this
+// takes 233; on one plane 424 and 406 us, 242 and 217 (before bins were split so
+// finely 724, 292; 733, 435).
+template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF, bool TEAMS>
+__global__ __launch_bounds__(64 * grid_mfma_max_waves<R>(),
+                             (grid_mfma_min_blocks<R, NPOL, MB, VB, COMP, TEAMS>()))
+void k_grid_mfma(PlanDev P, const R *__restrict__ vis, const R *__restrict__ weight,
+                 const uint8_t *__restrict__ flag, R *__restrict__ grid, int mode, int share,
+                 uint32_t most_alone) {
+  extern __shared__ __align__(16) char smem[];
+  const MfmaLds L = mfma_lds_layout<R, NPOL>(P.ov, P.support, 16 * (MB > VB ? MB : VB));
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t n_units = P.gunit_start[P.n_bins];
+  const auto copy_tables = [&]() {
+    copy_wtab_padded((R *)(smem + L.tab), L, P);
+    for (int i = tid; i < L.nnrm; i += blockDim.x) ((double *)(smem + L.nrm))[i] = P.nrm[i];
+    __syncthreads();
+  };
+  // 16 workgroups of 4 units: the 64 channels of a tile under one L2
+  const uint32_t units_per_wg = TEAMS ? max(share, 1) : blockDim.x / 64;
+  const uint32_t blk = xcd_grouped_block(blockIdx.x, kGridXcdGroup * kGridMaxWaves / units_per_wg);
+  if constexpr (!TEAMS) {
+    if (blk * units_per_wg >= n_units) return;  // whole workgroup idle
+    copy_tables();  // the only workgroup barrier
+    // the same for every lane: scalar registers for the unit and its bounds
+    const uint32_t u =
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)(blk * units_per_wg + wave));
+    if (u >= n_units || (COMP && (P.gunits[u].w & kUnitMulti))) return;
+    grid_mfma_unit<R, NPOL, MB, VB, COMP, PSF, TEAMS>(P, L, smem, vis, weight, flag, grid, mode, u,
+                                                      false);
+  } else {
+    // the workgroup's units: consecutive ones, or every gridDim.x-th, 64 at a time
+    const bool all = share > 0;
+    const uint32_t stride = all ? 1u : gridDim.x, per = all ? units_per_wg : 64u;
+    bool have_tables = false;
+    for (uint32_t at = all ? blk * per : blockIdx.x; at < n_units;
+         at += all ? n_units : 64 * stride) {
+      const uint32_t mine = at + lane * stride;
+      uint32_t n_in = 0;
+      if (lane < per && mine < n_units) {
+        const uint4 unit = P.gunits[mine];
+        uint32_t cnt;
+        bool multi;
+        if (!(unit.w & kUnitMulti))
+          n_in = all ? 1 : 0;
+        else if (!comp_group(P, unit.x, unit.y, n_in, cnt, multi))
+          n_in = 0;
+      }
+      // groups for one wavefront, and for all: the same in every wavefront
+      unsigned long long alone = __ballot(n_in > 0 && n_in <= most_alone);
+      unsigned long long teams = __ballot(n_in > most_alone);
+      if (!(alone | teams)) continue;
+      if (!have_tables) copy_tables();
+      have_tables = true;
+      // those for one in turn among the wavefronts
+      for (int k = 0; alone | teams;) {
+        const bool team = alone == 0;
+        unsigned long long &from = team ? teams : alone;
+        const uint32_t l = (uint32_t)__ffsll(from) - 1;
+        from &= from - 1;
+        if (!team && (k++ & (kGridMaxWaves - 1)) != wave) continue;
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)(at + l * stride));
+        grid_mfma_unit<R, NPOL, MB, VB, COMP, PSF, TEAMS>(P, L, smem, vis, weight, flag, grid, mode,
+                                                          u, team);
+      }
+    }
+  }
 }
 
 // Compensated mode, around the gridder: clear the FP64 slots of split bins
@@ -893,7 +974,7 @@ template <int NPOL, int MB, int VB, bool FINISH>
 __global__ __launch_bounds__(256) void k_comp_slots(PlanDev P, float *grid, int accumulate) {
   using MV = typename MfmaOp<float>::V;
   constexpr int C = 2 * NPOL, kNc = MB * C * VB * 4;
-  double *slots = comp_slots(P, mfma_comb_bytes<NPOL, MB, VB, true>());
+  double *slots = comp_slots(P, comp_slot_bytes<NPOL, MB, VB>());
   if (!slots) return;
   const uint32_t n_units = P.gunit_start[P.n_bins];
   const int lane = threadIdx.x & 63;
@@ -1057,12 +1138,29 @@ static int launch_grid(av_plan *plan, const void *vis, const void *weight, const
   return AV_OK;
 }
 
+// How a compensated call covers a plan's units: kFew, a workgroup per unit, when
+// they do not fill the chip (a 128^2 snapshot of two polarisations: 52 us, four
+// to a workgroup 59); kRare, where the samples could split few bins (a twelfth of
+// the bins or less), one launch without teams, whose registers leave a fifth more
+// wavefronts to a SIMD, and one for the split bins (13 M samples x 2 polarisations
+// on 64 planes of 2048^2: 2.13 ms, in one launch 3.08, a workgroup per unit 6.18;
+// 6.5 M on 16 planes of 1024^2, where a fifth of the bins could be split, 755 us,
+// 599 and 1043); else kMany, four units to a workgroup.
+constexpr int64_t kCompRareBins = 12;      // bins per unit of samples
+constexpr int64_t kCompGroupWgs = 8192;    // workgroups of the launch for split bins
+constexpr uint32_t kCompMostAlone = 2;     // units of a group that one wavefront takes
+enum class CompCover { kFew, kRare, kMany };
+static CompCover comp_cover(const PlanDev &d) {
+  if (d.max_gunits < kGridWideUnits) return CompCover::kFew;
+  return d.n_bins >= kCompRareBins * (d.n_items / d.unit_cap) ? CompCover::kRare
+                                                              : CompCover::kMany;
+}
+
 template <typename R, int NPOL, int MB, int VB, bool COMP, bool PSF>
 static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
                             const uint8_t *flag, const double *cgk, void *grid, double *sumwt,
                             int mode, hipStream_t s) {
   PlanDev &d = plan->d;
-  auto kfn = k_grid_mfma<R, NPOL, MB, VB, COMP, PSF>;
   const DeviceProps &prop = device_props();
   if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
   const MfmaLds L = mfma_lds_layout<R, NPOL>(d.ov, d.support, 16 * (MB > VB ? MB : VB));
@@ -1072,26 +1170,42 @@ static int launch_grid_mfma(av_plan *plan, const void *vis, const void *weight,
         (size_t)(L.st_d + kGridWideWaves * L.wave_bytes) <= prop.lds_per_block)
       nw = kGridWideWaves;
   }
-  const int lds = L.st_d + nw * L.wave_bytes + mfma_comb_bytes<NPOL, MB, VB, COMP>();
-  {
-    const int rc_lds = ensure_lds_limit<k_grid_mfma<R, NPOL, MB, VB, COMP, PSF>>(lds, "av_grid: hipFuncSetAttribute");
-    if (rc_lds) return rc_lds;
-  }
-  const unsigned nsb = (unsigned)std::max<int64_t>(
-      1, std::min<int64_t>((d.max_gunits + 255) / 256, 4096));
-  if constexpr (COMP) {
+  const int lds = L.st_d + nw * L.wave_bytes;
+  const auto launch = [&](auto teams, int64_t wgs, int share, uint32_t most_alone) {
+    constexpr bool kTeams = decltype(teams)::value;
+    const int rc = ensure_lds_limit<k_grid_mfma<R, NPOL, MB, VB, COMP, PSF, kTeams>>(
+        lds, "av_grid: hipFuncSetAttribute");
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_grid_mfma<R, NPOL, MB, VB, COMP, PSF, kTeams>), dim3((unsigned)wgs),
+                       dim3(64 * nw), lds, s, d, (const R *)vis, (const R *)weight, flag,
+                       (R *)grid, mode, share, most_alone);
+    AV_LAUNCH_CHECK("k_grid_mfma");
+    return AV_OK;
+  };
+  const auto grouped = [&](int units) {  // workgroups of `units` units
+    return xcd_grouped_grid((d.max_gunits + units - 1) / units,
+                            kGridXcdGroup * kGridMaxWaves / units);
+  };
+  int rc;
+  if constexpr (!COMP) {
+    if ((rc = launch(std::false_type{}, grouped(nw), 0, 1))) return rc;
+  } else {
+    const unsigned nsb = (unsigned)std::max<int64_t>(
+        1, std::min<int64_t>((d.max_gunits + 255) / 256, 4096));
     hipLaunchKernelGGL((k_comp_slots<NPOL, MB, VB, false>), dim3(nsb), dim3(256), 0, s, d,
                        (float *)grid, 0);
     AV_LAUNCH_CHECK("k_comp_slots");
-  }
-  const int units_per_wg = COMP ? 1 : nw;
-  const unsigned nwg =
-      (unsigned)xcd_grouped_grid((d.max_gunits + units_per_wg - 1) / units_per_wg,
-                                 kGridXcdGroup * kGridMaxWaves / units_per_wg);
-  hipLaunchKernelGGL(kfn, dim3(nwg), dim3(64 * nw), lds, s, d, (const R *)vis,
-                     (const R *)weight, flag, cgk, (R *)grid, mode);
-  AV_LAUNCH_CHECK("k_grid_mfma");
-  if constexpr (COMP) {
+    const CompCover cover = comp_cover(d);
+    if (cover == CompCover::kRare) {
+      if ((rc = launch(std::false_type{}, grouped(nw), 0, 1)) ||
+          (rc = launch(std::true_type{}, std::min<int64_t>((d.max_gunits + 3) / 4, kCompGroupWgs),
+                       0, kCompMostAlone)))
+        return rc;
+    } else {
+      const int share = cover == CompCover::kFew ? 1 : nw;
+      if ((rc = launch(std::true_type{}, grouped(share), share, share > 1 ? kCompMostAlone : 1)))
+        return rc;
+    }
     hipLaunchKernelGGL((k_comp_slots<NPOL, MB, VB, true>), dim3(nsb), dim3(256), 0, s, d,
                        (float *)grid, mode & AV_GRID_ACCUMULATE);
     AV_LAUNCH_CHECK("k_comp_slots");
@@ -1927,8 +2041,7 @@ static int try_mfma(av_plan *plan, const void *vis, const void *weight, const ui
       if (prop.error) return hip_fail(prop.error, "av_grid: device properties");
       const MfmaLds L = mfma_lds_layout<R, NPOL>(plan->d.ov, plan->d.support,
                                                  16 * (MB > VB ? MB : VB));
-      if ((size_t)L.total + mfma_comb_bytes<NPOL, MB, VB, COMP>() > prop.lds_per_block)
-        return AV_OK;
+      if ((size_t)L.total > prop.lds_per_block) return AV_OK;
       done = true;
       if (mode & AV_GRID_PSF)
         return launch_grid_mfma<R, NPOL, MB, VB, COMP, true>(plan, vis, weight, flag, cgk, grid,

@@ -393,8 +393,6 @@ def grid_kernel_name(tile, n_pol: int, fp64: bool = False, compensated: bool = F
         pad = max(tu, tv)
         up16 = lambda b: (b + 15) & ~15
         total = up16((support + 2 * pad) * nw * r) + up16(nw * 8) + 4 * (64 * 2 * n_pol * r + 64 * 8)
-        if compensated:  # FP64 tiles the wavefronts of a group add in
-            total += (tu // 16) * 2 * n_pol * (tv // 16) * 4 * 64 * 8
         if total <= lds_bytes:
             if (tu, tv) == (16, 16) and not fp64 and not compensated and not f32_products:
                 return "k_grid_h3"

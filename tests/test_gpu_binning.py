@@ -257,3 +257,41 @@ def test_degrid_units_longer_than_grid_units(gpu, nchan, prec):
     # 256 records a grid unit; as many, two and four times as many a degrid unit
     ratio = units[0][0] / units[0][1]
     assert ratio > {1: 1.0, 2: 1.8, 4: 3.0}[nchan]
+
+
+@pytest.mark.parametrize("npol", [1, 2, 4])
+@pytest.mark.parametrize("cap", [0, 64, 100, 4096, 8192])
+@pytest.mark.parametrize("n", [80, 1040])
+def test_compensated_sums_of_few_and_many_split_bins(gpu, oracle, n, cap, npol):
+    """Bins of one unit, of two, of several and of several groups, side by side
+    on a plan where most bins are split (80^2: 25 tiles) and on one where few
+    are (1040^2: 4225), the sums and their bounds as above."""
+    from astroviper_amd.device import GridPlan
+    tiles = (n // 16) ** 2
+    counts = np.full(tiles, 3)
+    counts[:8] = (13000, 9000, 5000, 700, 200, 150, 520, 64)
+    counts[-2:] = (8300, 129)
+    rng = np.random.default_rng(n + cap + npol)
+    at = np.repeat(np.arange(tiles), counts)
+    nt = n // 16
+    px = np.stack([16 * (at // nt), 16 * (at % nt)], 1) + 8 + rng.uniform(-4, 4, (at.size, 2))
+    px = px[rng.permutation(at.size)]
+    freq, cell = np.array([1.2e9]), 1e-4
+    scale = -(freq[0] * np.array([-cell, cell]) * n) / C
+    uvw = np.concatenate([(px - n // 2) / scale, np.zeros((at.size, 1))], 1)
+    w = rng.uniform(0.5, 1.5, (at.size, npol)).astype(np.float32)
+    gref, swref = oracle.standard_grid(None, uvw[:, None], w[:, None, None].astype(float), freq,
+                                       (n, n), (-cell, cell), chan_mode="cube", do_psf=True)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    plan = GridPlan(at.size, 1, 1, (n, n), (-cell, cell), unit_cap=cap, device=gpu)
+    plan.set_uvw(dev(uvw), dev(freq))
+    assert plan.stats()["records"] == at.size
+    g, sw = plan.grid(None, dev(w), psf=True, compensated=True)
+    assert _rel(g.cpu().numpy(), gref) < 8 * 2.0 ** -24
+    assert _rel(sw.cpu().numpy(), swref) < 1e-12
+    # small bins by themselves: beside the largest cell their errors would not show
+    tail = np.s_[..., -32:-16, :]
+    assert _rel(g.cpu().numpy()[tail], gref[tail]) < 8 * 2.0 ** -24
+    g, sw = plan.grid(None, dev(w), grid=g, sumwt=sw, psf=True, accumulate=True, compensated=True)
+    assert _rel(g.cpu().numpy(), 2 * gref) < 16 * 2.0 ** -24
+    plan.close()
