@@ -60,6 +60,9 @@ constexpr int kMosaicStage = 64;
 // units per XCD group: a tile's channels are consecutive units, so a group
 // of 64 keeps a tile's units (and the samples they share) on one XCD's L2
 constexpr uint32_t kMosaicGroup = 64;
+// kernel values are copied by phase for this many samples or more, and at most so
+// many values a sample (see launch_mosaic)
+constexpr int64_t kPhaseSamples = 1 << 17, kPhaseValues = 16;
 
 template <typename R>
 struct MosaicArgs {
@@ -90,8 +93,8 @@ struct MosaicArgs {
 // elements apart along v and ov_u * cv_n along u, so the 64 lanes of a load
 // touched 64 cache lines and the gridder waited on the vector L1, one line a
 // cycle; by phase they are rows of consecutive elements, about 6 lines a
-// load.  The copy is one pass over a table that k_mosaic_norms reads whole
-// anyway.
+// load.  The copy is one pass over the table, made where the samples are worth it
+// (launch_mosaic).
 template <typename R>
 __global__ __launch_bounds__(256) void k_mosaic_phases(MosaicArgs<R> A, int64_t total, R *out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -494,8 +497,12 @@ static int launch_mosaic(av_plan *plan, MosaicArgs<R> A, double *sumwt, int mode
   A.dv_lo = -(A.ov_v / 2) - 1;
   A.ndv = A.ov_v + 3;
   const int64_t entries = ncf * A.ndu * A.ndv;
-  // The kernel values by phase, unless the padded table reaches 2^31 elements
-  // or there is no room for it: then the caller's order is read
+  // The kernel values by phase where the samples are worth the pass over the
+  // table and it has room: else the caller's order is read.  Samples of 4
+  // channels x 2 polarisations on 1024^2, FP32, by phase and in order: 403 k
+  // and 0.1 M kernel values 328 and 339 us, 0.6 M 349 and 366, 4.8 M 389 and 399,
+  // 10.8 M 510 and 471, 1.6 M at oversampling 32 323 and 586; 97 k and 0.1 M
+  // 209 and 199, 10.8 M 388 and 246; 8 k and 10.8 M 216 and 102.
   const int64_t tu = ((int64_t)A.cu_n + A.ov_u - 1) / A.ov_u;
   const int64_t tv = ((int64_t)A.cv_n + A.ov_v - 1) / A.ov_v;
   A.taps_u = (int)tu;
@@ -503,7 +510,9 @@ static int launch_mosaic(av_plan *plan, MosaicArgs<R> A, double *sumwt, int mode
   A.last_u = (int)(A.cu_n - 1 - (tu - 1) * A.ov_u);
   A.last_v = (int)(A.cv_n - 1 - (tv - 1) * A.ov_v);
   const int64_t pad_u = tu * A.ov_u, pad_v = tv * A.ov_v;
-  const bool phases = pad_v < ((int64_t)1 << 31) / pad_u &&
+  const bool phases = d.n_items >= kPhaseSamples &&
+                      ncf * A.cu_n * A.cv_n <= kPhaseValues * d.n_items &&
+                      pad_v < ((int64_t)1 << 31) / pad_u &&
                       pad_u * pad_v < ((int64_t)1 << 31) / ncf;
   const int64_t pad = phases ? ncf * pad_u * pad_v : 0;
   // one stream-ordered block: the kernel sums, max(weight_support), then the
