@@ -8,14 +8,17 @@
 //   predict_model_visibilities applies it, imager.py:96-99): taper,
 //   real-to-complex FFT along v | FFT along u, the other half from
 //   F[-k] = conj(F[k]), fftshift.
-// What bounds them is memory: the grid and the image once, the half spectrum
-// in between written and read once.  32 planes of 2048 x 2048, complex64 to
-// FP64 images: 1.41 ms for 6.4 GB, 4.6 TB/s, the rate of a large copy here
-// (fold, rocFFT's complex-to-real transform and normalisation: 3.87 ms); 16
-// planes of 1024 x 1024 FP64: 0.20 ms (transform alone: 0.36).  Groups of
-// planes whose half spectra fit the 256 MB Infinity Cache were slower (1.58
-// ms in groups of two planes): their last workgroups leave more idle than the
-// cache saves.  The groups only bound the work memory.
+// What bounds them is memory, at two thirds to nine tenths of a large copy's 4.67
+// TB/s: the grid and the image once, the half spectrum in between written and
+// read once.  32 planes of 2048 x 2048, complex64 to FP64 images: 1.41 ms for 4.5
+// GB counted (columns 2.35, rows 2.15), 3.2 TB/s, as a block of long columns fills
+// a CU's LDS and no other workgroup loads while it computes (fold, rocFFT's
+// complex-to-real transform and normalisation: 3.87 ms); 16 planes of 1024 x 1024
+// FP64: 0.20 ms to the image for 0.71 GB, 3.5 TB/s, 0.17 to the grid for 0.74, 4.3
+// TB/s (transform alone: 0.36).  Groups of planes whose half spectra fit the 256 MB
+// Infinity Cache were slower (1.58 ms in groups of two planes): their last
+// workgroups leave more idle than the cache saves.  The groups only bound the work
+// memory.
 //
 // A workgroup transforms several columns (or rows) of one plane in LDS, in
 // FP64 whatever the types in memory.  The transform is Stockham's

@@ -62,7 +62,7 @@ constexpr int kMosaicStage = 64;
 constexpr uint32_t kMosaicGroup = 64;
 // kernel values are copied by phase for this many samples or more, and at most so
 // many values a sample (see launch_mosaic)
-constexpr int64_t kPhaseSamples = 1 << 17, kPhaseValues = 16;
+constexpr int64_t kPhaseSamples = 3 << 14, kPhaseValues = 32;
 
 template <typename R>
 struct MosaicArgs {
@@ -498,11 +498,12 @@ static int launch_mosaic(av_plan *plan, MosaicArgs<R> A, double *sumwt, int mode
   A.ndv = A.ov_v + 3;
   const int64_t entries = ncf * A.ndu * A.ndv;
   // The kernel values by phase where the samples are worth the pass over the
-  // table and it has room: else the caller's order is read.  Samples of 4
-  // channels x 2 polarisations on 1024^2, FP32, by phase and in order: 403 k
-  // and 0.1 M kernel values 328 and 339 us, 0.6 M 349 and 366, 4.8 M 389 and 399,
-  // 10.8 M 510 and 471, 1.6 M at oversampling 32 323 and 586; 97 k and 0.1 M
-  // 209 and 199, 10.8 M 388 and 246; 8 k and 10.8 M 216 and 102.
+  // table and it has room: else the caller's order is read.  By phase and in
+  // order, FP32: 8 k samples x 2 polarisations on 4 planes of 1024^2 and 0.1 M
+  // kernel values 88 and 80 us, 10.8 M 216 and 102; 97 k and 4.8 M 267 and 231, 1.6
+  // M at oversampling 32 204 and 232; 403 k and 0.1 M 328 and 339, 10.8 M 510 and
+  // 471 (FP64 810 and 866), 1.6 M at oversampling 32 323 and 586; 65 k samples on
+  // 32 planes of 768^2 and 0.1 M 168 and 183.
   const int64_t tu = ((int64_t)A.cu_n + A.ov_u - 1) / A.ov_u;
   const int64_t tv = ((int64_t)A.cv_n + A.ov_v - 1) / A.ov_v;
   A.taps_u = (int)tu;

@@ -60,9 +60,9 @@ def test_mosaic_polarisation_split(gpu, oracle, pol_maps, side, prec):
 
 @pytest.mark.parametrize("prec", [64, 32])
 @pytest.mark.parametrize("pol_maps,side,n_time", [
-    ([0], 47, 993),        # 131,076 samples: the fewest whose kernel values are copied by phase
-    ([0], 47, 992),        # one time fewer: read in the caller's order
-    ([1, 1], 47, 1000), ([1, 0], 5, 1000), ([0, 1, 1, 0], 47, 1000),
+    ([0], 47, 373),        # 49,236 samples: the fewest whose kernel values are copied by phase
+    ([0], 47, 372),        # one time fewer: read in the caller's order
+    ([1, 1], 47, 400), ([1, 0], 5, 400), ([0, 1, 1, 0], 47, 400),
 ])
 def test_mosaic_kernel_values_by_phase(gpu, oracle, pol_maps, side, n_time, prec):
     """Enough samples for kernel values by phase.  A cell sums some ten thousand
