@@ -120,7 +120,8 @@ int av_ps_outer(const double *k1, int32_t nrow, int32_t nfill,
  *             AV_PLAN_ROW_CHANNELS (then av_plan_set_uvw needs row_chan);
  *             AV_GEOM_REFERENCE may also be or'ed with AV_GEOM_CONJUGATE
  * unit_cap    records per work unit (0 = chosen from the number of samples,
- *             256 to 8192)
+ *             256 to 8192; degrid units then up to four times as long where
+ *             the plan has several image channels)
  * The plan is device-resident; create it once per (shape, tiling). */
 typedef struct av_plan av_plan;
 
